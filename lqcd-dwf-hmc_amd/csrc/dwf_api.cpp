@@ -3074,7 +3074,8 @@ struct dwf_smear_s {
   size_t V;
   std::vector<double*> levels;
   bool have_config = false;
-  double* itheta = nullptr;   // scratch of the force recursion (lazy)
+  std::vector<double*> chunked;   // levels 0 .. nsmear - 1 in chunked form
+  double* itheta = nullptr;       // scratch of the force recursion (lazy), chunked form
 };
 
 int dwf_smear_create(const int dims[4], double rho, int nsmear, dwf_smear* out) {
@@ -3094,6 +3095,12 @@ int dwf_smear_create(const int dims[4], double rho, int nsmear, dwf_smear* out) 
       dwf_smear_destroy(sm);
       return fail(DWF_ERR_HIP, "device allocation failed");
     }
+  sm->chunked.assign(nsmear, nullptr);
+  for (auto& l : sm->chunked)
+    if (hipMalloc(&l, gauge_chunked_bytes(sm->V)) != hipSuccess) {
+      dwf_smear_destroy(sm);
+      return fail(DWF_ERR_HIP, "device allocation failed");
+    }
   *out = sm;
   return DWF_OK;
 }
@@ -3102,14 +3109,18 @@ int dwf_smear_destroy(dwf_smear sm) {
   if (g_ctx.stream) (void)hipStreamSynchronize(g_ctx.stream);
   for (auto l : sm->levels)
     if (l) (void)hipFree(l);
+  for (auto l : sm->chunked)
+    if (l) (void)hipFree(l);
   if (sm->itheta) (void)hipFree(sm->itheta);
   delete sm;
   return DWF_OK;
 }
 static int smear_levels(dwf_smear sm) {
+  if (sm->nsmear > 0)
+    HIPCHK(launch_gauge_chunk(sm->chunked[0], sm->levels[0], sm->N, g_ctx.stream));
   for (int i = 0; i < sm->nsmear; ++i)
-    HIPCHK(launch_stout(sm->levels[i + 1], sm->levels[i], sm->N[0], sm->N[1], sm->N[2], sm->N[3],
-                        sm->rho, g_ctx.stream));
+    HIPCHK(launch_stout(sm->levels[i + 1], i + 1 < sm->nsmear ? sm->chunked[i + 1] : nullptr,
+                        sm->chunked[i], sm->N, sm->rho, g_ctx.stream));
   sm->have_config = true;
   return DWF_OK;
 }
@@ -3150,9 +3161,9 @@ int dwf_smear_force_udiv(dwf_smear sm, int level, double* Sigma, const double* S
   if (!sm || !Sigma || !Sigmap) return fail(DWF_ERR_INVALID_ARG, "null argument");
   if (level < 0 || level >= sm->nsmear) return fail(DWF_ERR_INVALID_ARG, "no such smearing level");
   if (!sm->have_config) return fail(DWF_ERR_NO_CONFIG, "set_config has not been called");
-  if (!sm->itheta) HIPCHK(hipMalloc(&sm->itheta, sm->V * 4 * 18 * sizeof(double)));
-  HIPCHK(launch_stout_force(Sigma, sm->itheta, Sigmap, sm->levels[level], sm->N[0], sm->N[1],
-                            sm->N[2], sm->N[3], sm->rho, g_ctx.stream));
+  if (!sm->itheta) HIPCHK(hipMalloc(&sm->itheta, gauge_chunked_bytes(sm->V)));
+  HIPCHK(launch_stout_force(Sigma, sm->itheta, Sigmap, sm->chunked[level], sm->N, sm->rho,
+                            g_ctx.stream));
   return DWF_OK;
 }
 // AForce_F_Smeared_alt::mult_jacobian (aforce_F_Smeared_alt-tmpl.h:170-191), in place

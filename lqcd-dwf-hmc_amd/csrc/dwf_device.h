@@ -192,4 +192,13 @@ struct Geo {
   int Ls;   // extent of the 5th dimension
 };
 
+// Workgroups are dispatched round-robin over the 8 XCDs (each with its own
+// L2).  Remap the hardware workgroup id so that every XCD walks a contiguous
+// range of sites: neighbouring sites then share an L2.
+__device__ __forceinline__ int xcd_block(int w, int G) {
+  const int q = G >> 3, r = G & 7;
+  const int x = w & 7, i = w >> 3;
+  return x * q + (x < r ? x : r) + i;
+}
+
 }  // namespace dwf

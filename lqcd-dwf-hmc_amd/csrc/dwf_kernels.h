@@ -280,14 +280,19 @@ hipError_t launch_chiral_gram(int prec, const void* const* fields, int F, int Vh
                               double* partial, double* out, hipStream_t st);
 size_t gram_partial_doubles();
 
-// Gauge: one stout smearing level, lexical Field_G (4, V, 18) double device.
-hipError_t launch_stout(double* Uout, const double* Uin, int Nx, int Ny, int Nz, int Nt,
-                        double rho, hipStream_t st);
+// Gauge fields, lexical Field_G (4, V, 18) double device, and their chunked form
+// (dwf_su3.h) that the smearing kernels read neighbour links from:
+size_t gauge_chunked_bytes(size_t V);
+hipError_t launch_gauge_chunk(double* Uc, const double* U, const int* dims, hipStream_t st);
+// one stout smearing level of the chunked links Uc, as a Field_G and, unless null,
+// in chunked form
+hipError_t launch_stout(double* Uout, double* Unext, const double* Uc, const int* dims, double rho,
+                        hipStream_t st);
 // One level of the stout force recursion: Sigma = dS/dU from Sigmap = dS/dU'
-// (U' = stout(U)); iTheta: scratch gauge field.  Lexical Field_G double device.
+// (U' = stout(U), U as the chunked Uc); Field_G both, Sigma may be Sigmap; iTheta:
+// scratch of gauge_chunked_bytes.
 hipError_t launch_stout_force(double* Sigma, double* iTheta, const double* Sigmap,
-                              const double* Uin, int Nx, int Ny, int Nz, int Nt, double rho,
-                              hipStream_t st);
+                              const double* Uc, const int* dims, double rho, hipStream_t st);
 // F <- -2 at(U F) over nlinks = 4 V links of a lexical gauge field U
 hipError_t launch_mult_generator_gauge(double* F, const double* U, size_t nlinks,
                                        hipStream_t st);

@@ -393,15 +393,6 @@ __device__ __forceinline__ void hop_all(C (*acc)[24], const T* __restrict__ in, 
 #endif
 }
 
-// Workgroups are dispatched round-robin over the 8 XCDs (each with its own
-// L2).  Remap the hardware workgroup id so that every XCD walks a contiguous
-// range of sites: neighbouring sites then share an L2.
-__device__ __forceinline__ int xcd_block(int w, int G) {
-  const int q = G >> 3, r = G & 7;
-  const int x = w & 7, i = w >> 3;
-  return x * q + (x < r ? x : r) + i;
-}
-
 // Matrix-core tile of the chiral epilogue: D(16x16) += A(16x4) B(4x16), lane l
 // holding A[l % 16][l / 16] and B[l / 16][l % 16].  Register r of lane l holds
 // D[4 (l / 16) + r][l % 16] for f32 and D[l / 16 + 4 r][l % 16] for f64 (both

@@ -68,56 +68,92 @@ __device__ M3 exp_iQ(const M3& iQ) {
   return r;
 }
 
-// C_mu(x) = rho sum_{nu != mu} (upper + lower staple)
-__device__ M3 staple_sum(const double* __restrict__ Uin, size_t site, int mu, size_t V, int Nx,
-                         int Ny, int Nz, int Nt, double rho) {
-  M3 Cst;
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) Cst.a[i][j] = {0, 0};
-  const size_t xpmu = shift_site(site, mu, +1, Nx, Ny, Nz, Nt);
-  for (int nu = 0; nu < 4; ++nu) {
-    if (nu == mu) continue;
-    const size_t xpnu = shift_site(site, nu, +1, Nx, Ny, Nz, Nt);
-    const size_t xmnu = shift_site(site, nu, -1, Nx, Ny, Nz, Nt);
-    const size_t xmnupmu = shift_site(xmnu, mu, +1, Nx, Ny, Nz, Nt);
-    // upper: U_nu(x) U_mu(x+nu) U_nu(x+mu)^+
-    const M3 up = mul_nn(load3(Uin + 18 * (site + V * nu)),
-                         mul_nd(load3(Uin + 18 * (xpnu + V * mu)), load3(Uin + 18 * (xpmu + V * nu))));
-    // lower: U_nu(x-nu)^+ U_mu(x-nu) U_nu(x-nu+mu)
-    const M3 lo = mul_dn(load3(Uin + 18 * (xmnu + V * nu)),
-                         mul_nn(load3(Uin + 18 * (xmnu + V * mu)), load3(Uin + 18 * (xmnupmu + V * nu))));
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        Cst.a[i][j].r += rho * up.a[i][j].r + rho * lo.a[i][j].r;
-        Cst.a[i][j].i += rho * up.a[i][j].i + rho * lo.a[i][j].i;
-      }
+// One wave per (mu, 64 consecutive sites), the four directions of a chunk next to
+// each other: their staples share links in L2.  From the chunked form these kernels
+// run at the 14.5 TB/s that gathers reach in L2 (19, 20 and 37 matrices per link at
+// 32x16x16x24: smearing 279 -> 159 us, force link part 358 -> 264, staple part 428 ->
+// 284); from the Field_G rows the L1's line lookups bound them, and gathering the
+// rows through LDS took 183, 330 and 320 us.
+struct GaugeWave {
+  int mu, first, lane;
+  dbl2v_t* sh;
+  __device__ __forceinline__ GaugeWave(dbl2v_t* slots) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int w = xcd_block(blockIdx.x, gridDim.x) * 2 + wave;
+    mu = w & 3;
+    first = (w >> 2) * 64;
+    lane = threadIdx.x & 63;
+    sh = slots + wave * kRowsLds;
   }
-  return Cst;
-}
+};
 
+// Field_G -> chunked form (see dwf_su3.h); 41 us at 32x16x16x24, a copy's time.
+template <bool WIDE>
 __global__ void __launch_bounds__(128)
-k_stout(double* __restrict__ Uout, const double* __restrict__ Uin, int Nx, int Ny, int Nz,
-        int Nt, double rho) {
-  const size_t V = (size_t)Nx * Ny * Nz * Nt;
-  const size_t idx = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  if (idx >= 4 * V) return;
-  const int mu = (int)(idx / V);
-  const size_t site = idx - (size_t)mu * V;
-  const M3 Cst = staple_sum(Uin, site, mu, V, Nx, Ny, Nz, Nt, rho);
-  const M3 U = load3(Uin + 18 * (site + V * mu));
-  const M3 iQ = at3(mul_nd(Cst, U));
-  store3(Uout + 18 * (site + V * mu), mul_nn(exp_iQ(iQ), U));
+k_gauge_chunk(double* __restrict__ Uc, const double* __restrict__ U, GaugeLat L) {
+  __shared__ dbl2v_t slots[2 * kRowsLds];
+  const GaugeWave g(slots);
+  const M3 m = rows_load<WIDE>(U + (size_t)18 * L.V * g.mu, g.first, L.V, g.sh);
+  store3c(reinterpret_cast<dbl2v_t*>(Uc) + chunked_mu(L) * g.mu, g.first + g.lane, m);
 }
 
-hipError_t launch_stout(double* Uout, const double* Uin, int Nx, int Ny, int Nz, int Nt,
-                        double rho, hipStream_t st) {
-  const size_t n = 4 * (size_t)Nx * Ny * Nz * Nt;
-  hipLaunchKernelGGL(k_stout, dim3((unsigned)((n + 127) / 128)), dim3(128), 0, st, Uout, Uin,
-                     Nx, Ny, Nz, Nt, rho);
+// C_mu(x) = rho sum_{nu != mu} (upper + lower staple), U in chunked form
+__device__ __forceinline__ M3 staple_sum(const double* __restrict__ Uc, const GaugeLat& L,
+                                         const GaugeSite& x, int mu, double rho) {
+  const size_t vol = chunked_mu(L);
+  const dbl2v_t* u0 = reinterpret_cast<const dbl2v_t*>(Uc);
+  const dbl2v_t* um = u0 + vol * mu;
+  const int pm = x.off(L, mu, 1);
+  M3 C = m3_zero();
+  for (int i = 0; i < 3; ++i) {
+    const int nu = i + (i >= mu ? 1 : 0);
+    const dbl2v_t* un = u0 + vol * nu;
+    const int pn = x.off(L, nu, 1), mn = x.off(L, nu, -1);
+    // upper: U_nu(x) [U_mu(x+nu) U_nu(x+mu)^+]
+    M3 t = mul_nd(load3c(um, x.s + pn), load3c(un, x.s + pm));
+    m3_axpy(C, rho, mul_nn(load3c(un, x.s), t));
+    // lower: U_nu(x-nu)^+ [U_mu(x-nu) U_nu(x-nu+mu)]
+    t = mul_nn(load3c(um, x.s + mn), load3c(un, x.s + mn + pm));
+    m3_axpy(C, rho, mul_dn(load3c(un, x.s + mn), t));
+  }
+  return C;
+}
+
+// One smearing level from the chunked links; Unext: the same level in chunked form
+// for the one after it (nullptr: not wanted).
+template <bool WIDE>
+__global__ void __launch_bounds__(128, 2)
+k_stout(double* __restrict__ Uout, double* __restrict__ Unext, const double* __restrict__ Uc,
+        GaugeLat L, double rho) {
+  __shared__ dbl2v_t slots[2 * kRowsLds];
+  const GaugeWave g(slots);
+  const GaugeSite x(L, g.first + g.lane);
+  const M3 C = staple_sum(Uc, L, x, g.mu, rho);
+  const M3 U = load3c(reinterpret_cast<const dbl2v_t*>(Uc) + chunked_mu(L) * g.mu, x.s);
+  const M3 iQ = at3(mul_nd(C, U));
+  const M3 V = mul_nn(exp_iQ(iQ), U);
+  if (Unext) store3c(reinterpret_cast<dbl2v_t*>(Unext) + chunked_mu(L) * g.mu, g.first + g.lane, V);
+  rows_store<WIDE>(Uout + (size_t)18 * L.V * g.mu, g.first, L.V, g.sh, V);
+}
+
+size_t gauge_chunked_bytes(size_t V) { return chunked_doubles(V) * sizeof(double); }
+
+hipError_t launch_gauge_chunk(double* Uc, const double* U, const int* dims, hipStream_t st) {
+  const GaugeLat L = gauge_lat(dims);
+  const dim3 grid(2 * L.chunks), block(128);
+  if (m3_wide(U)) hipLaunchKernelGGL(k_gauge_chunk<true>, grid, block, 0, st, Uc, U, L);
+  else hipLaunchKernelGGL(k_gauge_chunk<false>, grid, block, 0, st, Uc, U, L);
+  return hipGetLastError();
+}
+
+hipError_t launch_stout(double* Uout, double* Unext, const double* Uc, const int* dims, double rho,
+                        hipStream_t st) {
+  const GaugeLat L = gauge_lat(dims);
+  const dim3 grid(2 * L.chunks), block(128);
+  if (m3_wide(Uout))
+    hipLaunchKernelGGL(k_stout<true>, grid, block, 0, st, Uout, Unext, Uc, L, rho);
+  else
+    hipLaunchKernelGGL(k_stout<false>, grid, block, 0, st, Uout, Unext, Uc, L, rho);
   return hipGetLastError();
 }
 
@@ -145,6 +181,15 @@ __device__ __forceinline__ M3 m3_poly(cplx c0, cplx c1, cplx c2, const M3& Q, co
 __device__ __forceinline__ cplx m3_tr(const M3& x) {
   return cadd(cadd(x.a[0][0], x.a[1][1]), x.a[2][2]);
 }
+// tr(x y)
+__device__ __forceinline__ cplx m3_trm(const M3& x, const M3& y) {
+  cplx s = {0.0, 0.0};
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) s = cadd(s, cmul(x.a[i][j], y.a[j][i]));
+  return s;
+}
 __device__ __forceinline__ cplx cexp_i(double phi) { return {cos(phi), sin(phi)}; }
 
 __device__ double stout_xi1(double w) {
@@ -156,36 +201,32 @@ __device__ double stout_xi1(double w) {
   return (w * cos(w) - sin(w)) / (w * w * w);
 }
 
-__global__ void __launch_bounds__(128)
-k_stout_force_link(double* __restrict__ Sigma, double* __restrict__ iTheta,
-                   const double* __restrict__ Sigmap, const double* __restrict__ Uin, int Nx,
-                   int Ny, int Nz, int Nt, double rho) {
-  const size_t V = (size_t)Nx * Ny * Nz * Nt;
-  const size_t idx = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  if (idx >= 4 * V) return;
-  const int mu = (int)(idx / V);
-  const size_t site = idx - (size_t)mu * V;
-  const size_t off = 18 * (site + V * mu);
-  const M3 C = staple_sum(Uin, site, mu, V, Nx, Ny, Nz, Nt, rho);
-  const M3 U = load3(Uin + off);
-  const M3 Sp = load3(Sigmap + off);
-  const M3 iQ = at3(mul_nd(C, U));
+template <bool WIDE>
+__global__ void __launch_bounds__(128, 2)
+k_stout_force_link(double* Sigma, double* __restrict__ iTheta, const double* Sigmap,
+                   const double* __restrict__ Uc, GaugeLat L, double rho) {
+  __shared__ dbl2v_t slots[2 * kRowsLds];
+  const GaugeWave gw(slots);
+  const GaugeSite x(L, gw.first + gw.lane);
+  const size_t off = (size_t)18 * L.V * gw.mu, offc = chunked_mu(L) * gw.mu;
+  const M3 C = staple_sum(Uc, L, x, gw.mu, rho);
+  const dbl2v_t* ul = reinterpret_cast<const dbl2v_t*>(Uc) + offc;
+  M3 iQ, US;
+  {
+    const M3 U = load3c(ul, x.s);
+    iQ = at3(mul_nd(C, U));
+    US = mul_nn(U, rows_load<WIDE>(Sigmap + off, gw.first, L.V, gw.sh));
+  }
   double n2 = 0;
 #pragma unroll
   for (int i = 0; i < 3; ++i)
 #pragma unroll
     for (int j = 0; j < 3; ++j) n2 += iQ.a[i][j].r * iQ.a[i][j].r + iQ.a[i][j].i * iQ.a[i][j].i;
-  M3 eiQ, iGam;
+  M3 eiQ = m3_zero(), iGam = m3_zero();
 #pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      eiQ.a[i][j] = {i == j ? 1.0 : 0.0, 0.0};
-      iGam.a[i][j] = {0.0, 0.0};
-    }
+  for (int i = 0; i < 3; ++i) eiQ.a[i][i].r = 1.0;
   if (n2 > 1.0e-10) {
     const M3 iQ2 = mul_nn(iQ, iQ);
-    const M3 iQ3 = mul_nn(iQ, iQ2);
     M3 Q, Q2;   // Q = -i iQ, Q^2 = -iQ^2
 #pragma unroll
     for (int i = 0; i < 3; ++i)
@@ -194,7 +235,8 @@ k_stout_force_link(double* __restrict__ Sigma, double* __restrict__ iTheta,
         Q.a[i][j] = {iQ.a[i][j].i, -iQ.a[i][j].r};
         Q2.a[i][j] = {-iQ2.a[i][j].r, -iQ2.a[i][j].i};
       }
-    const double c0 = -(iQ3.a[0][0].i + iQ3.a[1][1].i + iQ3.a[2][2].i) / 3.0;
+    const double q3 = m3_trm(iQ, iQ2).i;
+    const double c0 = -(q3) / 3.0;
     const double c1 = -0.5 * (iQ2.a[0][0].r + iQ2.a[1][1].r + iQ2.a[2][2].r);
     const double c13r = sqrt(c1 / 3.0);
     const double ratio = fmin(1.0, fmax(-1.0, c0 / (2.0 * c13r * c13r * c13r)));
@@ -233,12 +275,14 @@ k_stout_force_link(double* __restrict__ Sigma, double* __restrict__ iTheta,
     auto bj2 = [&](cplx ra, cplx rb, cplx f) {
       return cscal(bd, cadd(cadd(ra, cscal(-3.0 * u, rb)), cscal(-24.0 * u, f)));
     };
-    const M3 US = mul_nn(U, Sp);
-    const cplx t1 = m3_tr(mul_nn(US, m3_poly(bj1(r01, r02, f0), bj1(r11, r12, f1),
-                                             bj1(r21, r22, f2), Q, Q2)));
-    const cplx t2 = m3_tr(mul_nn(US, m3_poly(bj2(r01, r02, f0), bj2(r11, r12, f1),
-                                             bj2(r21, r22, f2), Q, Q2)));
-    const M3 QUS = mul_nn(Q, US), USQ = mul_nn(US, Q);
+    // tr(U S' B_j), B_j = b_j0 + b_j1 Q + b_j2 Q^2
+    const M3 USQ = mul_nn(US, Q);
+    const cplx s0 = m3_tr(US), s1 = m3_tr(USQ), s2 = m3_trm(US, Q2);
+    const cplx t1 = cadd(cadd(cmul(bj1(r01, r02, f0), s0), cmul(bj1(r11, r12, f1), s1)),
+                         cmul(bj1(r21, r22, f2), s2));
+    const cplx t2 = cadd(cadd(cmul(bj2(r01, r02, f0), s0), cmul(bj2(r11, r12, f1), s1)),
+                         cmul(bj2(r21, r22, f2), s2));
+    const M3 QUS = mul_nn(Q, US);
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -251,81 +295,74 @@ k_stout_force_link(double* __restrict__ Sigma, double* __restrict__ iTheta,
     eiQ = m3_poly(f0, f1, f2, Q, Q2);
   }
   const M3 iLam = at3(iGam);
-  store3(iTheta + off, mul_nn(iLam, U));
+  // U and S' are read again (from L2) rather than kept: holding them spills
+  asm volatile("" : "+s"(ul));
+  const M3 U = load3c(ul, x.s);
+  const M3 Sp = rows_load<WIDE>(Sigmap + off, gw.first, L.V, gw.sh);
+  store3c(reinterpret_cast<dbl2v_t*>(iTheta) + offc, gw.first + gw.lane, mul_nn(iLam, U));
   M3 Xi = mul_nn(Sp, eiQ);
-  const M3 CdL = mul_dn(C, iLam);
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) Xi.a[i][j] = cadd(Xi.a[i][j], CdL.a[i][j]);
-  store3(Sigma + off, Xi);
+  m3_add(Xi, mul_dn(C, iLam));
+  rows_store<WIDE>(Sigma + off, gw.first, L.V, gw.sh, Xi);
 }
 
 // Sigma_mu(x) += rho sum_{nu != mu} of the six staple products (force_each,
-// aforceSmear_APE-tmpl.h:280-360)
-__global__ void __launch_bounds__(128)
-k_stout_force_staple(double* __restrict__ Sigma, const double* __restrict__ Uin,
-                     const double* __restrict__ iTheta, int Nx, int Ny, int Nz, int Nt,
-                     double rho) {
-  const size_t V = (size_t)Nx * Ny * Nz * Nt;
-  const size_t idx = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  if (idx >= 4 * V) return;
-  const int mu = (int)(idx / V);
-  const size_t site = idx - (size_t)mu * V;
-  auto Ul = [&](size_t s, int d) { return load3(Uin + 18 * (s + V * d)); };
-  auto Th = [&](size_t s, int d) { return load3(iTheta + 18 * (s + V * d)); };
-  M3 acc;
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) acc.a[i][j] = {0, 0};
-  const size_t xpmu = shift_site(site, mu, +1, Nx, Ny, Nz, Nt);
-  for (int nu = 0; nu < 4; ++nu) {
-    if (nu == mu) continue;
-    const size_t xpnu = shift_site(site, nu, +1, Nx, Ny, Nz, Nt);
-    const size_t xmnu = shift_site(site, nu, -1, Nx, Ny, Nz, Nt);
-    const size_t xmnupmu = shift_site(xmnu, mu, +1, Nx, Ny, Nz, Nt);
-    const M3 Vnu_xpmu = Ul(xpmu, nu), Vmu_xpnu = Ul(xpnu, mu), Vnu_x = Ul(site, nu);
-    const M3 Vnu_b = Ul(xmnupmu, nu), Vmu_mn = Ul(xmnu, mu), Vnu_mn = Ul(xmnu, nu);
-    // forward-staple products (x, x+mu, x+nu)
-    const M3 a = mul_nd(Vnu_xpmu, Vmu_xpnu);                       // V_nu(x+mu) V_mu(x+nu)^+
-    M3 t = mul_nd(a, Th(site, nu));                                // ... iTheta_nu(x)^+
-    const M3 t4 = mul_nd(mul_nd(Th(xpmu, nu), Vmu_xpnu), Vnu_x);   // iTheta_nu(x+mu) V_mu(x+nu)^+ V_nu(x)^+
-    const M3 t6 = mul_nd(mul_nd(Vnu_xpmu, Th(xpnu, mu)), Vnu_x);   // V_nu(x+mu) iTheta_mu(x+nu)^+ V_nu(x)^+
-    // backward-staple products (x-nu, x-nu+mu)
-    const M3 t2 = mul_nn(mul_dn(Vnu_b, dag3(Th(xmnu, mu))), Vnu_mn);  // V_nu^+ iTheta_mu^+ V_nu
-    const M3 b = mul_dn(Vnu_b, dag3(Vmu_mn));                          // V_nu(x-nu+mu)^+ V_mu(x-nu)^+
-    const M3 t3 = mul_nn(b, Th(xmnu, nu));                             // ... iTheta_nu(x-nu)
-    const M3 t5 = mul_nn(mul_dn(Th(xmnupmu, nu), dag3(Vmu_mn)), Vnu_mn); // iTheta_nu^+ V_mu^+ V_nu
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        cplx v = cadd(cadd(t.a[i][j], t2.a[i][j]), cadd(t3.a[i][j], t4.a[i][j]));
-        v = cadd(v, cadd(t5.a[i][j], t6.a[i][j]));
-        acc.a[i][j] = cadd(acc.a[i][j], cscal(rho, v));
-      }
+// aforceSmear_APE-tmpl.h:280-360), V the links and T = iTheta, two of the three
+// products of each side sharing a factor:
+//   [T_nu(x+mu) V_mu(x+nu)^+ + V_nu(x+mu) T_mu(x+nu)^+] V_nu(x)^+
+//     + V_nu(x+mu) V_mu(x+nu)^+ T_nu(x)^+
+//   [V_nu(b)^+ T_mu(m)^+ + T_nu(b)^+ V_mu(m)^+] V_nu(m) + V_nu(b)^+ V_mu(m)^+ T_nu(m),
+// m = x-nu, b = x-nu+mu. 
+template <bool WIDE>
+__global__ void __launch_bounds__(128, 2)
+k_stout_force_staple(double* __restrict__ Sigma, const double* __restrict__ Uc,
+                     const double* __restrict__ iTheta, GaugeLat L, double rho) {
+  __shared__ dbl2v_t slots[2 * kRowsLds];
+  const GaugeWave g(slots);
+  const int mu = g.mu;
+  const GaugeSite x(L, g.first + g.lane);
+  const size_t vol = chunked_mu(L);
+  const dbl2v_t* u0 = reinterpret_cast<const dbl2v_t*>(Uc);
+  const dbl2v_t* t0 = reinterpret_cast<const dbl2v_t*>(iTheta);
+  const dbl2v_t *vm = u0 + vol * mu, *tm = t0 + vol * mu;
+  const int pm = x.off(L, mu, 1);
+  M3 acc = m3_zero();
+  for (int i = 0; i < 3; ++i) {
+    const int nu = i + (i >= mu ? 1 : 0);
+    const dbl2v_t *vn = u0 + vol * nu, *tn = t0 + vol * nu;
+    const int pn = x.off(L, nu, 1), m = x.s + x.off(L, nu, -1), b = m + pm;
+    {
+      const M3 Vn = load3c(vn, x.s + pm), Vm = load3c(vm, x.s + pn);
+      m3_axpy(acc, rho, mul_nd(mul_nd(Vn, Vm), load3c(tn, x.s)));
+      M3 t = mul_nd(load3c(tn, x.s + pm), Vm);
+      m3_add(t, mul_nd(Vn, load3c(tm, x.s + pn)));
+      m3_axpy(acc, rho, mul_nd(t, load3c(vn, x.s)));
+    }
+    const M3 Vb = load3c(vn, b), Vm = load3c(vm, m);
+    m3_axpy(acc, rho, mul_nn(mul_dd(Vb, Vm), load3c(tn, m)));
+    M3 t = mul_dd(Vb, load3c(tm, m));
+    m3_add(t, mul_dd(load3c(tn, b), Vm));
+    m3_axpy(acc, rho, mul_nn(t, load3c(vn, m)));
   }
-  double* out = Sigma + 18 * (site + V * mu);
-  M3 s0 = load3(out);
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) s0.a[i][j] = cadd(s0.a[i][j], acc.a[i][j]);
-  store3(out, s0);
+  double* out = Sigma + (size_t)18 * L.V * mu;
+  m3_add(acc, rows_load<WIDE>(out, g.first, L.V, g.sh));
+  rows_store<WIDE>(out, g.first, L.V, g.sh, acc);
 }
 
 hipError_t launch_stout_force(double* Sigma, double* iTheta, const double* Sigmap,
-                              const double* Uin, int Nx, int Ny, int Nz, int Nt, double rho,
-                              hipStream_t st) {
-  const size_t n = 4 * (size_t)Nx * Ny * Nz * Nt;
-  const dim3 grid((unsigned)((n + 127) / 128));
-  hipLaunchKernelGGL(k_stout_force_link, grid, dim3(128), 0, st, Sigma, iTheta, Sigmap, Uin, Nx,
-                     Ny, Nz, Nt, rho);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_stout_force_staple, grid, dim3(128), 0, st, Sigma, Uin,
-                     (const double*)iTheta, Nx, Ny, Nz, Nt, rho);
+                              const double* Uc, const int* dims, double rho, hipStream_t st) {
+  const GaugeLat L = gauge_lat(dims);
+  const dim3 grid(2 * L.chunks), block(128);
+  if (m3_wide(Sigma, Sigmap)) {
+    hipLaunchKernelGGL(k_stout_force_link<true>, grid, block, 0, st, Sigma, iTheta, Sigmap, Uc, L,
+                       rho);
+    hipLaunchKernelGGL(k_stout_force_staple<true>, grid, block, 0, st, Sigma, Uc,
+                       (const double*)iTheta, L, rho);
+  } else {
+    hipLaunchKernelGGL(k_stout_force_link<false>, grid, block, 0, st, Sigma, iTheta, Sigmap, Uc, L,
+                       rho);
+    hipLaunchKernelGGL(k_stout_force_staple<false>, grid, block, 0, st, Sigma, Uc,
+                       (const double*)iTheta, L, rho);
+  }
   return hipGetLastError();
 }
 
