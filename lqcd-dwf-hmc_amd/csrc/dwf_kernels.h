@@ -260,11 +260,13 @@ hipError_t launch_ms_fold(void* const* x, void* const* p, const void* const* R,
 hipError_t launch_lincomb(void* v, const void* b, double a0, void* const* x, const double* c,
                           int m, size_t n, hipStream_t st);
 
-// Force: F_mu(x) (+)= scale * sum_{s,d} [(1 + sgn g_mu) Vn(x+mu) bc]_{a,d,s} conj(Z(x)_{b,d,s})
-// for the sites x of one parity; F lexical Field_G (4, V, 18) double.
-hipError_t launch_force_tensor(double* F, const double* Z, const double* Vn, const int* nbr,
-                               int parity, int Nx, int Ny, int Nz, int Nt, const int* bc,
-                               int Ls, double sgn, double scale, bool accumulate,
+// Force, both parities: F_mu(x) (+)= scale * sum_{s,d} of
+//   terms & 1: [(1 - g_mu) y(x+mu) bc]_{a,d,s} conj(b(x)_{b,d,s})
+//   terms & 2: [(1 + g_mu) b(x+mu) bc]_{a,d,s} conj(y(x)_{b,d,s})
+// b, y: the fields of parity 0 and 1; F lexical Field_G (4, V, 18) double.
+hipError_t launch_force_tensor(double* F, int terms, const double* const* b,
+                               const double* const* y, const int* nbr, const int* N,
+                               const int* bc, int Ls, double scale, bool accumulate,
                                hipStream_t st);
 // F <- -2 at(U F) with U from the packed forward links
 hipError_t launch_mult_generator(double* F, const double* links, int Nx, int Ny, int Nz, int Nt,

@@ -65,48 +65,6 @@ size_t prec_bytes(int prec) {
   }
 }
 
-// ---------------------------------------------------------------------------
-// spin projection / reconstruction, Dirac basis.  dir = 2*mu + fb,
-// fb = 0: (1 - gamma_mu) U_mu(x) psi(x+mu), fb = 1: (1 + gamma_mu) U^+ psi(x-mu).
-// w[k], k = ri + 2*(c + 3*d).
-// ---------------------------------------------------------------------------
-template <int DIR, typename C>
-__device__ __forceinline__ void project(const C* w, C* h1, C* h2) {
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    const int r = 2 * c, i = 2 * c + 1;
-    const C* w0 = w;
-    const C* w1 = w + 6;
-    const C* w2 = w + 12;
-    const C* w3 = w + 18;
-    if (DIR == 0) {         // h1 = w0 + i w3, h2 = w1 + i w2
-      h1[r] = w0[r] - w3[i]; h1[i] = w0[i] + w3[r];
-      h2[r] = w1[r] - w2[i]; h2[i] = w1[i] + w2[r];
-    } else if (DIR == 1) {  // h1 = w0 - i w3, h2 = w1 - i w2
-      h1[r] = w0[r] + w3[i]; h1[i] = w0[i] - w3[r];
-      h2[r] = w1[r] + w2[i]; h2[i] = w1[i] - w2[r];
-    } else if (DIR == 2) {  // h1 = w0 + w3, h2 = w1 - w2
-      h1[r] = w0[r] + w3[r]; h1[i] = w0[i] + w3[i];
-      h2[r] = w1[r] - w2[r]; h2[i] = w1[i] - w2[i];
-    } else if (DIR == 3) {  // h1 = w0 - w3, h2 = w1 + w2
-      h1[r] = w0[r] - w3[r]; h1[i] = w0[i] - w3[i];
-      h2[r] = w1[r] + w2[r]; h2[i] = w1[i] + w2[i];
-    } else if (DIR == 4) {  // h1 = w0 + i w2, h2 = w1 - i w3
-      h1[r] = w0[r] - w2[i]; h1[i] = w0[i] + w2[r];
-      h2[r] = w1[r] + w3[i]; h2[i] = w1[i] - w3[r];
-    } else if (DIR == 5) {  // h1 = w0 - i w2, h2 = w1 + i w3
-      h1[r] = w0[r] + w2[i]; h1[i] = w0[i] - w2[r];
-      h2[r] = w1[r] - w3[i]; h2[i] = w1[i] + w3[r];
-    } else if (DIR == 6) {  // h1 = 2 w2, h2 = 2 w3
-      h1[r] = w2[r] + w2[r]; h1[i] = w2[i] + w2[i];
-      h2[r] = w3[r] + w3[r]; h2[i] = w3[i] + w3[i];
-    } else {                // h1 = 2 w0, h2 = 2 w1
-      h1[r] = w0[r] + w0[r]; h1[i] = w0[i] + w0[i];
-      h2[r] = w1[r] + w1[r]; h2[i] = w1[i] + w1[i];
-    }
-  }
-}
-
 template <int DIR, typename C>
 __device__ __forceinline__ void reconstruct(C* o, const C* a1, const C* a2) {
 #pragma unroll

@@ -311,7 +311,7 @@ k_stout_force_link(double* Sigma, double* __restrict__ iTheta, const double* Sig
 //   [T_nu(x+mu) V_mu(x+nu)^+ + V_nu(x+mu) T_mu(x+nu)^+] V_nu(x)^+
 //     + V_nu(x+mu) V_mu(x+nu)^+ T_nu(x)^+
 //   [V_nu(b)^+ T_mu(m)^+ + T_nu(b)^+ V_mu(m)^+] V_nu(m) + V_nu(b)^+ V_mu(m)^+ T_nu(m),
-// m = x-nu, b = x-nu+mu. 
+// m = x-nu, b = x-nu+mu.
 template <bool WIDE>
 __global__ void __launch_bounds__(128, 2)
 k_stout_force_staple(double* __restrict__ Sigma, const double* __restrict__ Uc,
