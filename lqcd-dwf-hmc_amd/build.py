@@ -20,7 +20,7 @@ CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "dwf_amd", "libdwfhip.so")
 OBJ = os.path.join(HERE, "_build")
 
-SOURCES = ["dwf_kernels.hip", "dwf_smear.hip", "dwf_force.hip", "dwf_lpc.hip", "dwf_batch.hip",
+SOURCES = ["dwf_kernels.hip", "dwf_small.hip", "dwf_smear.hip", "dwf_force.hip", "dwf_lpc.hip", "dwf_batch.hip",
            "dwf_hmc.hip", "dwf_ptc.hip", "dwf_rng.cpp", "dwf_io.cpp", "dwf_api.cpp"]
 
 HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")

@@ -243,4 +243,43 @@ __device__ __forceinline__ void project(const C* w, C* h1, C* h2) {
   }
 }
 
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+  return v;
+}
+
+// Sum of n partials by one block of up to 8 waves, in a fixed order (thread t
+// adds t, t + blockDim, ...; then the wave sums in wave order); with 256
+// threads it is the order of k_red_finish.  sh holds 8 doubles.
+__device__ __forceinline__ double block_sum(const double* __restrict__ p, unsigned n,
+                                            double* sh) {
+  double w = 0;
+  for (unsigned i = threadIdx.x; i < n; i += blockDim.x) w += p[i];
+  const double t = wave_sum(w);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = t;
+  __syncthreads();
+  double r = 0;
+  for (unsigned k = 0; k < (blockDim.x >> 6); ++k) r += sh[k];
+  __syncthreads();
+  return r;
+}
+
+// a = U h for a 3x3 row-major complex matrix u[ab], ab = ri + 2*(b + 3*a)
+template <typename C>
+__device__ __forceinline__ void su3_mul(const C* u, const C* h, C* a) {
+#pragma unroll
+  for (int ia = 0; ia < 3; ++ia) {
+    C re = 0, im = 0;
+#pragma unroll
+    for (int ib = 0; ib < 3; ++ib) {
+      const C ur = u[2 * (ib + 3 * ia)], ui = u[2 * (ib + 3 * ia) + 1];
+      re += ur * h[2 * ib] - ui * h[2 * ib + 1];
+      im += ur * h[2 * ib + 1] + ui * h[2 * ib];
+    }
+    a[2 * ia] = re;
+    a[2 * ia + 1] = im;
+  }
+}
+
 }  // namespace dwf

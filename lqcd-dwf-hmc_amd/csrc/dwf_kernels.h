@@ -66,6 +66,12 @@ struct Epi {
   size_t rstride = 0;
 };
 
+// The same launch by the small-lattice kernel (dwf_small.hip), and the rule for it.
+bool small_dwf_applies(int prec, int op, int Vh, int Ls, const Epi& e);
+hipError_t launch_dwf_small(int prec, int op, void* out, const void* in, const void* links,
+                            const int* nbr, int parity, int Vh, int Ls, const Epi& e,
+                            hipStream_t st, unsigned* nblocks);
+
 // Grouped launch: up to kGroupMax lattices (same Ls, precision and epilogue
 // form; compile-time Ls 12 or 16; FP64 or FP32) in one launch of the fused
 // kernel.  The member table lives in device memory and is built once.

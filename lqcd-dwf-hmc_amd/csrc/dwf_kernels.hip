@@ -35,28 +35,6 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-  return v;
-}
-
-// Sum of n partials by one block of up to 8 waves, in a fixed order (thread t
-// adds t, t + blockDim, ...; then the wave sums in wave order); with 256
-// threads it is the order of k_red_finish.  sh holds 8 doubles.
-__device__ __forceinline__ double block_sum(const double* __restrict__ p, unsigned n,
-                                            double* sh) {
-  double w = 0;
-  for (unsigned i = threadIdx.x; i < n; i += blockDim.x) w += p[i];
-  const double t = wave_sum(w);
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = t;
-  __syncthreads();
-  double r = 0;
-  for (unsigned k = 0; k < (blockDim.x >> 6); ++k) r += sh[k];
-  __syncthreads();
-  return r;
-}
-
 size_t prec_bytes(int prec) {
   switch (prec) {
     case P64: return 8;
@@ -119,23 +97,6 @@ __device__ __forceinline__ void su3_mul2_lds(const C* up, int stride, const C* h
     a1[2 * ia + 1] = i1;
     a2[2 * ia] = r2;
     a2[2 * ia + 1] = i2;
-  }
-}
-
-// a = U h for a 3x3 row-major complex matrix u[ab], ab = ri + 2*(b + 3*a)
-template <typename C>
-__device__ __forceinline__ void su3_mul(const C* u, const C* h, C* a) {
-#pragma unroll
-  for (int ia = 0; ia < 3; ++ia) {
-    C re = 0, im = 0;
-#pragma unroll
-    for (int ib = 0; ib < 3; ++ib) {
-      const C ur = u[2 * (ib + 3 * ia)], ui = u[2 * (ib + 3 * ia) + 1];
-      re += ur * h[2 * ib] - ui * h[2 * ib + 1];
-      im += ur * h[2 * ib + 1] + ui * h[2 * ib];
-    }
-    a[2 * ia] = re;
-    a[2 * ia + 1] = im;
   }
 }
 
@@ -1355,7 +1316,9 @@ hipError_t launch_dwf(int prec, int op, void* out, const void* in, const void* l
                       hipStream_t st) {
   hipError_t err = hipErrorInvalidValue;
   unsigned nb = 0;
-  switch (prec) {
+  if (small_dwf_applies(prec, op, Vh, Ls, e))
+    err = launch_dwf_small(prec, op, out, in, links, nbr, parity, Vh, Ls, e, st, &nb);
+  else switch (prec) {
     case P64: err = launch_dwf_t<double>(op, out, in, links, nbr, parity, Vh, Ls, e, st, &nb); break;
     case P32: err = launch_dwf_t<float>(op, out, in, links, nbr, parity, Vh, Ls, e, st, &nb); break;
     case P16: err = launch_dwf_t<__half>(op, out, in, links, nbr, parity, Vh, Ls, e, st, &nb); break;
