@@ -20,6 +20,7 @@
 // layout of the operator, element ((site * 24 + k) * Ls + s), k = ri + 2 (c + 3 d).
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 
 #include "dwf_device.h"
 #include "dwf_kernels.h"
@@ -165,25 +166,68 @@ __device__ __forceinline__ float ptc_ld(__amdgpu_buffer_rsrc_t r, unsigned voff,
   return __uint_as_float(ptc_ldu(r, voff, soff));
 }
 
+typedef unsigned ptc_w2_t __attribute__((ext_vector_type(2)));
+typedef short ptc_s4_t __attribute__((ext_vector_type(4)));
+
+// t = hi + mid + lo exactly, each part with at most 8 significant bits, i.e. a
+// bfloat16 (the first sixteen bits of its float): truncate, subtract, truncate.  The
+// parts of (re, im) are returned as one word each, re low; the subtraction takes its
+// part from the word (v_dot2_f32_bf16 with (-1, 0) and (0, -1), exact here).
+__device__ __forceinline__ void ptc_split(float re, float im, unsigned& hi, unsigned& mid,
+                                          unsigned& lo) {
+  typedef __bf16 b2_t __attribute__((ext_vector_type(2)));
+  constexpr unsigned kHigh = 0x07060302u;   // the upper halves of both
+  // kept in registers: as an inline constant the instruction reads -1.0 differently
+  unsigned kre = 0x0000bf80u, kim = 0xbf800000u;
+  asm("" : "+s"(kre), "+s"(kim));
+  const b2_t mre = __builtin_bit_cast(b2_t, kre), mim = __builtin_bit_cast(b2_t, kim);
+  auto top = [&](float x, float y) {
+    return __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), kHigh);
+  };
+  auto minus = [&](float x, unsigned w, b2_t m) {
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(b2_t, w), m, x, false);
+  };
+  hi = top(re, im);
+  const float re1 = minus(re, hi, mre), im1 = minus(im, hi, mim);
+  mid = top(re1, im1);
+  lo = top(minus(re1, mid, mre), minus(im1, mid, mim));
+}
+
 // Matrix-core form of the same layer (any number of output channels up to 16;
 // an odd count leaves the second channel of the last tile with zero weights and
 // does not store it).  Per path q and input channel b the contraction is the
 // real product
 //   [out_re; out_im](a, alpha) += [Wr -Wi; Wi Wr](a, alpha; beta) [t_re; t_im](beta)
-// for every colour, computed as v_mfma_f32_16x16x4f32 tiles D(16x16) +=
-// A(16x4) B(4x16) with
+// for every colour.  The weights are bfloat16, and the FP32 transports are the exact sum
+// of three bfloat16 parts, so the products run on the BF16 matrix cores without loss
+// (v_mfma_f32_16x16x16_bf16, FP32 accumulation): 3 x 16 cycles per tile, colour and two
+// input channels where the FP32 cores take 4 x 32.  Tiles D(16x16) += A(16x16) B(16x16) with
 //   D rows  m = 8 a' + 2 alpha + re/im  (NMT tiles of two output channels),
-//   K       beta (4 spins), one product for t_re and one for t_im,
+//   K       (spin beta, input channel b or b + 1, re/im), one product per part,
 //   columns 16 points (site, s) of one parity, consecutive in site * Ls + s.
-// Lane l holds A[l % 16][l / 16] and B[l / 16][l % 16], so lane l computes
+// Lane l holds A[l % 16][4 (l / 16) + i] and B[4 (l / 16) + i][l % 16], so lane l computes
 // the transport of spin beta = l / 16 at point l % 16 itself (3 colours, 36
-// multiply-adds for a hop path) and holds the weight of row l % 16, column
-// beta; register r of its result holds D[4 (l / 16) + r][l % 16].  One wave
+// multiply-adds for a hop path) and holds the weights of row l % 16, column
+// beta, which are the weight's own word for t: (Wr, -Wi) in a re row, (Wi, Wr) in an im
+// row; register r of its result holds D[4 (l / 16) + r][l % 16].  One wave
 // per 16 points, all output channels; each output element is a sum over
-// (q, b) of 4-spin matrix-core products in FP32.
-// three waves per SIMD (at most 168 registers) fit without spills up to NMT = 5
-template <bool ADJ, int NMT>
-__global__ void __launch_bounds__(256, NMT <= 5 ? 3 : 2)
+// (q, b pairs, parts) of 8-term matrix-core products in FP32.
+// 1 -> 8 -> 8 -> 8 -> 1 channels at 16^3 x 32, Ls = 16: 13.5 -> 8.8 ms (error against
+// 64 bits 9.5e-7 -> 6e-7).  Bound by the gathers: every channel is read nine times through
+// L1 (14.5 GB per 8 -> 8 layer, 12.6 GB of it past the L2s); the vector unit has 1.4 ms
+// of work per such layer (36 operations of transport and 21 of splitting per hop path
+// and channel), the matrix cores 1.35 ms.  Two s per lane with eight-byte loads (9.9 ms),
+// all channels per path (9.9) and no per-XCD order (9.6, before the shifts by lane, against
+// 9.6) were no faster.
+// The paths are the inner loop and the channel pairs the outer one: the points in flight
+// on an XCD then gather from two channels at a time, which its L2 holds between the nine
+// uses better than all of them.  The links of the wave's sites sit in LDS (they are read
+// once per pair), and so do the layer's weights where they fit (LW).  S16: Ls = 16, where
+// a tile is one site and the shifts in s are row shifts (DPP) of the split words.
+constexpr int kPtcLinkDir = 20, kPtcLinkSite = 8 * kPtcLinkDir;   // floats in LDS
+__host__ __device__ constexpr int ptc_wave_sites(int Ls) { return 15 / Ls + 2; }
+template <bool ADJ, int NMT, bool LW, bool S16>
+__global__ void __launch_bounds__(256, NMT <= 2 ? 4 : NMT <= 5 ? 3 : 2)
 k_ptc_layer_mfma(float* __restrict__ out, const float* __restrict__ in, int cin, int cout,
                  const unsigned* __restrict__ W, int wcin, int wcout,
                  const float* __restrict__ links, const int* __restrict__ nbr, int Vh, int Ls) {
@@ -192,133 +236,205 @@ k_ptc_layer_mfma(float* __restrict__ out, const float* __restrict__ in, int cin,
   // whose source is outside the lattice or the fifth dimension reads at
   // kOut and gets 0.  The launcher checks that every offset fits.
   constexpr unsigned kOut = 0x80000000u;
+  extern __shared__ __align__(16) unsigned ptc_sw[];
   const int lane = threadIdx.x & 63;
   const int n = lane & 15, g = lane >> 4;
   const size_t fsz = (size_t)Vh * 24 * Ls;
   const int npts = Vh * Ls;            // points of one parity
   const int tpp = (npts + 15) / 16;    // tiles of one parity
-  const int wpb = blockDim.x >> 6;
-  const unsigned lsb = 4u * (unsigned)Ls, vhb = 4u * (unsigned)Vh;
-  const __amdgpu_buffer_rsrc_t rl = ptc_rsrc(links, (unsigned)(2 * 8 * 18) * vhb);
-  const __amdgpu_buffer_rsrc_t rw =
-      ptc_rsrc(W, 4u * (unsigned)(kPtcPaths * wcin * wcout * 16));
+  const unsigned lsb = 4u * (unsigned)Ls;
+  const int nwords = kPtcPaths * wcin * wcout * 16;
+  const __amdgpu_buffer_rsrc_t rw = ptc_rsrc(W, 4u * (unsigned)nwords);
+  const int wsites = ptc_wave_sites(Ls);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  float* su = reinterpret_cast<float*>(ptc_sw) + (size_t)wave * wsites * kPtcLinkSite;
+  unsigned* sw = ptc_sw + (size_t)4 * wsites * kPtcLinkSite;
+  if (LW) {
+    for (int i = threadIdx.x; i < nwords / 4; i += 256)
+      reinterpret_cast<u32x4_t*>(sw)[i] = reinterpret_cast<const u32x4_t*>(W)[i];
+    __syncthreads();
+  }
   // the A row of this lane: channel 2 mt + am, spin row al, re (0) / im (1);
   // its weight word within the (q, b, mt) block
   const int am = n >> 3, al = (n >> 1) & 3, ro = n & 1;
+  // its word (Wr, Wi) as the coefficients of (t_re, t_im): halves exchanged in an im row,
+  // one sign (conjugated for the adjoint)
+  const unsigned wsel = ro ? 0x01000302u : 0x03020100u;
+  const unsigned wmask = ADJ ? (ro ? 0x8000u : 0u) : (ro ? 0u : 0x80000000u);
   const unsigned wlane =
-      4u * (ADJ ? (unsigned)(am * 16 + g * 4 + al) : (unsigned)(am * wcin * 16 + al * 4 + g));
-  for (int tile = blockIdx.x * wpb + (threadIdx.x >> 6); tile < 2 * tpp;
-       tile += gridDim.x * wpb) {
-    const int p = tile / tpp;
-    const int P = (tile - p * tpp) * 16 + n;
-    const bool valid = P < npts;
-    const int Pc = valid ? P : npts - 1;
-    const int site = Pc / Ls, s = Pc - (Pc / Ls) * Ls;
-    flt4_t acc[NMT][3];
+      ADJ ? (unsigned)(am * 16 + g * 4 + al) : (unsigned)(am * wcin * 16 + al * 4 + g);
+  // every XCD walks a contiguous range of sites: the neighbours of a tile share its L2
+  const int tile = xcd_block(blockIdx.x, gridDim.x) * 4 + wave;
+  if (tile >= 2 * tpp) return;
+  const int p = tile / tpp;
+  const int P0 = (tile - p * tpp) * 16, P = P0 + n;
+  const bool valid = P < npts;
+  const int Pc = valid ? P : npts - 1;
+  const int site = Pc / Ls, s = Pc - (Pc / Ls) * Ls;
+  // links of sites site0 .. site0 + wsites - 1 (those below Vh), [site][dir][20]
+  const int site0 = P0 / Ls;
+  for (int i = lane; i < 144 * wsites; i += 64) {
+    const int r = i / wsites, j = i - r * wsites, d = r / 18;   // row = dir * 18 + e
+    const int x = site0 + j < Vh ? site0 + j : Vh - 1;
+    su[j * kPtcLinkSite + d * kPtcLinkDir + (r - 18 * d)] =
+        links[((size_t)p * 144 + r) * Vh + x];
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const float* ul = su + (site - site0) * kPtcLinkSite;
+  // byte offsets of spin g of the source points in a channel
+  const unsigned own = 4u * (unsigned)(p * fsz + ((size_t)site * 24 + 6 * g) * Ls + s);
+  unsigned off[kPtcPaths];
+  off[0] = valid ? own : kOut;
 #pragma unroll
-    for (int mt = 0; mt < NMT; ++mt)
+  for (int d = 0; d < 8; ++d) {
+    const int nb = nbr[((size_t)p * 8 + d) * Vh + site];
+    off[1 + d] = valid ? 4u * (unsigned)((1 - p) * fsz + ((size_t)nb * 24 + 6 * g) * Ls + s) : kOut;
+  }
+  off[9] = valid && s + 1 < Ls ? own + 4u : kOut;
+  off[10] = valid && s > 0 ? own - 4u : kOut;
+  flt4_t acc[NMT][3];
 #pragma unroll
-      for (int c = 0; c < 3; ++c) acc[mt][c] = flt4_t{0.f, 0.f, 0.f, 0.f};
-    for (int q = 0; q < kPtcPaths; ++q) {
+  for (int mt = 0; mt < NMT; ++mt)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) acc[mt][c] = flt4_t{0.f, 0.f, 0.f, 0.f};
+  for (int b = 0; b < cin; b += 2) {
+    // the spinors of input channels b and b + 1 at the source points of path q, loaded one
+    // path ahead of the matrix-core products; a channel beyond cin reads zeros
+    const bool two = b + 1 < cin;
+    const __amdgpu_buffer_rsrc_t r0 = ptc_rsrc(in + (size_t)b * 2 * fsz, 8u * (unsigned)fsz);
+    const __amdgpu_buffer_rsrc_t r1 =
+        ptc_rsrc(in + (size_t)(two ? b + 1 : b) * 2 * fsz, two ? 8u * (unsigned)fsz : 0u);
+    auto load = [&](int q, float (&w)[2][6]) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) w[0][k] = ptc_ld(r0, off[q], (unsigned)k * lsb);
+#pragma unroll
+      for (int k = 0; k < 6; ++k) w[1][k] = ptc_ld(r1, off[q], (unsigned)k * lsb);
+    };
+    // element (al, beta = g) of the applied spin matrix of channel a = 2 mt + am:
+    // forward W[qw][a][b], adjoint (W[qw][b][a])^+, as the coefficients of (re, im);
+    // an odd cout pads the last tile, an odd cin the last pair with zeros
+    auto weights = [&](int q, ptc_w2_t (&A)[NMT]) {
       const int qw = ADJ ? ptc_rev(q) : q;   // weight path
-      const bool hop = q >= 1 && q <= 8;
+#pragma unroll
+      for (int mt = 0; mt < NMT; ++mt)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const unsigned wblk = ADJ ? (unsigned)(((qw * wcout + b + j) * wcin + 2 * mt) * 16)
+                                    : (unsigned)(((qw * wcout + 2 * mt) * wcin + b + j) * 16);
+          const bool on = (j == 0 || two) && 2 * mt + am < cout;
+          unsigned e;
+          if constexpr (LW) {
+            e = sw[on ? wblk + wlane : 0u];
+            e = on ? e : 0u;
+          } else {
+            e = ptc_ldu(rw, on ? 4u * wlane : kOut, 4u * wblk);
+          }
+          A[mt][j] = __builtin_amdgcn_perm(e, e, wsel) ^ wmask;
+        }
+    };
+    // the products of colour c, the parts in order of size
+    auto products = [&](const ptc_w2_t (&A)[NMT], const ptc_w2_t (&B)[3], int c) {
+#pragma unroll
+      for (int part = 0; part < 3; ++part)
+#pragma unroll
+        for (int mt = 0; mt < NMT; ++mt)
+          acc[mt][c] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+              __builtin_bit_cast(ptc_s4_t, A[mt]), __builtin_bit_cast(ptc_s4_t, B[part]),
+              acc[mt][c], 0, 0, 0);
+    };
+    auto split = [&](float re, float im, ptc_w2_t (&B)[3], int j) {
+      unsigned hi, mid, lo;
+      ptc_split(re, im, hi, mid, lo);
+      B[0][j] = lo;
+      B[1][j] = mid;
+      B[2][j] = hi;
+    };
+    // paths without a link
+    auto plain = [&](int q, const float (&w)[2][6]) {
+      ptc_w2_t A[NMT];
+      weights(q, A);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        ptc_w2_t B[3];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) split(w[j][2 * c], w[j][2 * c + 1], B, j);
+        products(A, B, c);
+        if constexpr (S16) {   // s + 1 and s - 1: the neighbouring lanes, 0 beyond the walls
+          ptc_w2_t U[3], D[3], Au[NMT], Ad[NMT];
+          weights(9, Au);
+          weights(10, Ad);
+#pragma unroll
+          for (int part = 0; part < 3; ++part)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+              U[part][j] = __builtin_amdgcn_update_dpp(0, (int)B[part][j], 0x101, 0xf, 0xf, true);
+              D[part][j] = __builtin_amdgcn_update_dpp(0, (int)B[part][j], 0x111, 0xf, 0xf, true);
+            }
+          products(Au, U, c);
+          products(Ad, D, c);
+        }
+      }
+    };
+    // a hop: colour by colour the transported component of spin g at this point, both
+    // channels, split, then its products
+    auto hop = [&](int q, const float (&w)[2][6]) {
+      ptc_w2_t A[NMT];
+      weights(q, A);
       float u[18];
-      unsigned woff;   // byte offset of spin g of the source point in a channel
-      if (hop) {
-        const int dir = q - 1;
-        const int nb = nbr[((size_t)p * 8 + dir) * Vh + site];
-        const unsigned loff = 4u * (unsigned)(((p * 8 + dir) * 18) * Vh + site);
 #pragma unroll
-        for (int e = 0; e < 18; ++e) u[e] = ptc_ld(rl, loff, (unsigned)e * vhb);
-        woff = valid ? 4u * (unsigned)((1 - p) * fsz + ((size_t)nb * 24 + 6 * g) * Ls + s) : kOut;
-      } else {
-        const int ss = q == 0 ? s : (q == 9 ? s + 1 : s - 1);
-        woff = valid && ss >= 0 && ss < Ls
-                   ? 4u * (unsigned)(p * fsz + ((size_t)site * 24 + 6 * g) * Ls + ss)
-                   : kOut;
+      for (int e = 0; e < 18; ++e) u[e] = ul[(q - 1) * kPtcLinkDir + e];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        ptc_w2_t B[3];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          float re = 0.f, im = 0.f;
+#pragma unroll
+          for (int cb = 0; cb < 3; ++cb)
+            cmac(re, im, u[2 * (cb + 3 * c)], u[2 * (cb + 3 * c) + 1], w[j][2 * cb],
+                 w[j][2 * cb + 1]);
+          split(re, im, B, j);
+        }
+        products(A, B, c);
       }
-      // the spinor of input channel b at the source point and this lane's
-      // weight words; loaded one channel ahead of the matrix-core products
-      auto load = [&](int b, float (&w)[6], unsigned (&e)[NMT]) {
-        const __amdgpu_buffer_rsrc_t ri = ptc_rsrc(in + (size_t)b * 2 * fsz, 8u * (unsigned)fsz);
-#pragma unroll
-        for (int k = 0; k < 6; ++k) w[k] = ptc_ld(ri, woff, (unsigned)k * lsb);
-        // element (al, beta = g) of the applied spin matrix of channel
-        // a = 2 mt + am: forward W[qw][a][b], adjoint (W[qw][b][a])^+
-#pragma unroll
-        for (int mt = 0; mt < NMT; ++mt) {
-          const unsigned wblk = ADJ ? (unsigned)(((qw * wcout + b) * wcin + 2 * mt) * 16)
-                                    : (unsigned)(((qw * wcout + 2 * mt) * wcin + b) * 16);
-          // an odd cout pads the last tile with a zero channel
-          e[mt] = ptc_ldu(rw, 2 * mt + am < cout ? wlane : kOut, 4u * wblk);
-        }
-      };
-      float wn[6];
-      unsigned en[NMT];
-      load(0, wn, en);
-      for (int b = 0; b < cin; ++b) {
-        float w[6];
-        unsigned e[NMT];
-#pragma unroll
-        for (int k = 0; k < 6; ++k) w[k] = wn[k];
-#pragma unroll
-        for (int mt = 0; mt < NMT; ++mt) e[mt] = en[mt];
-        if (b + 1 < cin) load(b + 1, wn, en);
-        float ar[NMT], ai[NMT];
-#pragma unroll
-        for (int mt = 0; mt < NMT; ++mt) {
-          const float wr = __uint_as_float(e[mt] << 16);
-          const float wi = ADJ ? -__uint_as_float(e[mt] & 0xffff0000u)
-                               : __uint_as_float(e[mt] & 0xffff0000u);
-          ar[mt] = ro ? wi : wr;    // multiplies t_re
-          ai[mt] = ro ? wr : -wi;   // multiplies t_im
-        }
-        // B operand: the transported colour vector of spin g at this point
-        float t[6];
-        if (hop) {
-#pragma unroll
-          for (int ca = 0; ca < 3; ++ca) {
-            float re = 0.f, im = 0.f;
-#pragma unroll
-            for (int cb = 0; cb < 3; ++cb)
-              cmac(re, im, u[2 * (cb + 3 * ca)], u[2 * (cb + 3 * ca) + 1], w[2 * cb],
-                   w[2 * cb + 1]);
-            t[2 * ca] = re;
-            t[2 * ca + 1] = im;
-          }
-        } else {
-#pragma unroll
-          for (int k = 0; k < 6; ++k) t[k] = w[k];
-        }
-#pragma unroll
-        for (int c = 0; c < 3; ++c)
-#pragma unroll
-          for (int mt = 0; mt < NMT; ++mt)
-            acc[mt][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(ar[mt], t[2 * c], acc[mt][c], 0, 0, 0);
-#pragma unroll
-        for (int c = 0; c < 3; ++c)
-#pragma unroll
-          for (int mt = 0; mt < NMT; ++mt)
-            acc[mt][c] =
-                __builtin_amdgcn_mfma_f32_16x16x4f32(ai[mt], t[2 * c + 1], acc[mt][c], 0, 0, 0);
-      }
+    };
+    float wa[2][6], wb[2][6];
+    load(0, wa);
+    if constexpr (S16) {
+      load(1, wb); plain(0, wa);
+      load(2, wa);
+    } else {
+      load(9, wb);  plain(0, wa);
+      load(10, wa); plain(9, wb);
+      load(1, wb);  plain(10, wa);
+      load(2, wa);
     }
-    if (valid) {
-      // register r: row 4 g + r = channel 2 mt + (g >> 1), spin 2 (g & 1) + (r >> 1),
-      // re / im r & 1
+    hop(1, wb); load(3, wb);
+    hop(2, wa); load(4, wa);
+    hop(3, wb); load(5, wb);
+    hop(4, wa); load(6, wa);
+    hop(5, wb); load(7, wb);
+    hop(6, wa); load(8, wa);
+    hop(7, wb);
+    hop(8, wa);
+  }
+  if (valid) {
+    // register r: row 4 g + r = channel 2 mt + (g >> 1), spin 2 (g & 1) + (r >> 1),
+    // re / im r & 1
 #pragma unroll
-      for (int mt = 0; mt < NMT; ++mt) {
-        if (2 * mt + (g >> 1) >= cout) continue;
-        float* o = out + (size_t)(2 * mt + (g >> 1)) * 2 * fsz + (size_t)p * fsz +
-                   (size_t)site * 24 * Ls + s;
+    for (int mt = 0; mt < NMT; ++mt) {
+      if (2 * mt + (g >> 1) >= cout) continue;
+      float* o = out + (size_t)(2 * mt + (g >> 1)) * 2 * fsz + (size_t)p * fsz +
+                 (size_t)site * 24 * Ls + s;
 #pragma unroll
-        for (int c = 0; c < 3; ++c)
+      for (int c = 0; c < 3; ++c)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int alo = 2 * (g & 1) + (r >> 1);
-            o[(size_t)((r & 1) + 2 * (c + 3 * alo)) * Ls] = acc[mt][c][r];
-          }
-      }
+        for (int r = 0; r < 4; ++r) {
+          const int alo = 2 * (g & 1) + (r >> 1);
+          o[(size_t)((r & 1) + 2 * (c + 3 * alo)) * Ls] = acc[mt][c][r];
+        }
     }
   }
 }
@@ -447,15 +563,24 @@ static void ptc_layer_launch(float* out, const float* in, int cin, int cout, con
                      links, nbr, Vh, Ls);
 }
 
+// weights in LDS where they and the links of the four waves fit in 64 KB
 template <bool ADJ, int NMT>
 static void ptc_layer_mfma_launch(float* out, const float* in, int cin, int cout,
                                   const unsigned* W, int wcin, int wcout, const float* links,
                                   const int* nbr, int Vh, int Ls, hipStream_t st) {
   const size_t tiles = 2 * (((size_t)Vh * Ls + 15) / 16);
-  size_t blocks = (tiles + 3) / 4;
-  if (blocks > 8192) blocks = 8192;
-  hipLaunchKernelGGL((k_ptc_layer_mfma<ADJ, NMT>), dim3((unsigned)blocks), dim3(256), 0, st, out,
-                     in, cin, cout, W, wcin, wcout, links, nbr, Vh, Ls);
+  const size_t wbytes = (size_t)kPtcPaths * wcin * wcout * 64;
+  const size_t lbytes = (size_t)4 * ptc_wave_sites(Ls) * kPtcLinkSite * sizeof(float);
+  const dim3 grid((unsigned)((tiles + 3) / 4)), block(256);
+  const bool lw = lbytes + wbytes <= 64 * 1024 && reinterpret_cast<uintptr_t>(W) % 16 == 0;
+#define PTC_GO(L, S)                                                                          \
+  hipLaunchKernelGGL((k_ptc_layer_mfma<ADJ, NMT, L, S>), grid, block, lbytes + (L ? wbytes : 0), \
+                     st, out, in, cin, cout, W, wcin, wcout, links, nbr, Vh, Ls)
+  if (lw && Ls == 16) PTC_GO(true, true);
+  else if (lw) PTC_GO(true, false);
+  else if (Ls == 16) PTC_GO(false, true);
+  else PTC_GO(false, false);
+#undef PTC_GO
 }
 
 template <bool ADJ>
