@@ -3368,10 +3368,7 @@ int dwf_ptc_loss_grad(dwf_ptc n, int nbatch, const void* const* b, const void* c
     int cur = 0;
     for (int l = L - 1; l >= 0; --l) {
       const int cin = n->ch[l], cout = n->ch[l + 1];
-      // block count: about 1024 lattice points per block, at most nblk
-      const size_t pts = (size_t)2 * op->Vh * op->Ls;
-      const int nbk = (int)std::max<size_t>(1, std::min<size_t>(n->nblk, pts / 1024));
-      HIPCHK(launch_ptc_wgrad(n->G, n->partial, nbk, n->g[cur], n->act[l], cin, cout,
+      HIPCHK(launch_ptc_wgrad(n->G, n->partial, n->nblk, n->g[cur], n->act[l], cin, cout,
                               (const float*)op->links, op->nbr, op->Vh, op->Ls, st));
       const size_t ng = (size_t)11 * cin * cout * 32;
       hG.resize(ng);

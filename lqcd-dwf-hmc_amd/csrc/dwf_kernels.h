@@ -145,7 +145,7 @@ hipError_t launch_finish_partials(int nr, const double* partial, unsigned nblock
 hipError_t launch_ptc_layer(bool adj, float* out, const float* in, int cin, int cout,
                             const unsigned short* W, int wcin, int wcout, const float* links,
                             const int* nbr, int Vh, int Ls, hipStream_t st);
-hipError_t launch_ptc_wgrad(double* G, double* partial, int nblk, const float* g, const float* in,
+hipError_t launch_ptc_wgrad(double* G, double* partial, int maxblk, const float* g, const float* in,
                             int cin, int cout, const float* links, const int* nbr, int Vh, int Ls,
                             hipStream_t st);
 hipError_t launch_ptc_embed(float* act, const float* x, size_t n, hipStream_t st);

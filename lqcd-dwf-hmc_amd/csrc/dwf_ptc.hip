@@ -193,6 +193,28 @@ __device__ __forceinline__ void ptc_split(float re, float im, unsigned& hi, unsi
   lo = top(minus(re1, mid, mre), minus(im1, mid, mim));
 }
 
+// The same split with rounded parts (their signs are then as good as random, so that a
+// dropped product of parts leaves no bias); a float within half a bfloat16 step of the
+// largest becomes infinite.
+__device__ __forceinline__ void ptc_split_round(float x, float y, unsigned& hi, unsigned& mid,
+                                                unsigned& lo) {
+  typedef __bf16 b2_t __attribute__((ext_vector_type(2)));
+  typedef float f2_t __attribute__((ext_vector_type(2)));
+  unsigned kx = 0x0000bf80u, ky = 0xbf800000u;
+  asm("" : "+s"(kx), "+s"(ky));
+  auto pack = [](float p, float q) { return __builtin_convertvector(f2_t{p, q}, b2_t); };
+  auto minus = [](float p, b2_t w, unsigned m) {
+    return __builtin_amdgcn_fdot2_f32_bf16(w, __builtin_bit_cast(b2_t, m), p, false);
+  };
+  const b2_t h = pack(x, y);
+  const float x1 = minus(x, h, kx), y1 = minus(y, h, ky);
+  const b2_t m = pack(x1, y1);
+  const b2_t l = pack(minus(x1, m, kx), minus(y1, m, ky));
+  hi = __builtin_bit_cast(unsigned, h);
+  mid = __builtin_bit_cast(unsigned, m);
+  lo = __builtin_bit_cast(unsigned, l);
+}
+
 // Matrix-core form of the same layer (any number of output channels up to 16;
 // an odd count leaves the second channel of the last tile with zero weights and
 // does not store it).  Per path q and input channel b the contraction is the
@@ -504,6 +526,239 @@ k_ptc_wgrad(double* __restrict__ partial, const float* __restrict__ g,
   }
 }
 
+// The same for Ls a multiple of 4 on the matrix cores: per path one real product
+//   P(64 x 64) = sum over points, colours of  g(a, alpha, re/im) t(b, beta, re/im)
+// with both operands split into three bfloat16 parts (rounded, so that what is left out has
+// no bias).  Six of the nine part products are taken, two at a time, as one
+// v_mfma_f32_16x16x32_bf16 per pair (K = 16 points x 2 parts): (hi lo)(lo hi),
+// (mid hi)(hi mid), (mid hi)(mid hi); the others are 2^-25 of a product and below, and with
+// (mid lo)(lo mid) the error against 64 bits is the same.  A block of four waves takes 16
+// points at a time (a lane four consecutive s of one component: 16-byte loads): wave w
+// loads, transports and splits the operands of row tile w and column tile w (a tile: two
+// channels) into LDS, then multiplies a quadrant of the 4 x 4 tiles; the sums over 16
+// points are added up in FP64.  Grid: blocks of points, paths, groups of 4 x 4 tiles.
+// Bound by the serial chain of a group (gather, transport, split, LDS, products, two
+// barriers: 3.4 us with three blocks per CU), neither by issue (fewer moves or address
+// instructions change nothing) nor by memory (nor does an order in which the paths share
+// an L2).  8 -> 8 channels at 8^3 x 16, Ls = 16: 1290 -> 507 us.
+__global__ void __launch_bounds__(256, 3)
+k_ptc_wgrad_mfma(double* __restrict__ partial, const float* __restrict__ gr,
+                 const float* __restrict__ in, int cin, int cout,
+                 const float* __restrict__ links, const int* __restrict__ nbr, int Vh, int Ls) {
+  typedef __bf16 b8_t __attribute__((ext_vector_type(8)));
+  // [tile][colour][part hi, mid, lo][lane]: any two parts are one conflict-free ds_read2_b64
+  __shared__ u32x2_t shA[4 * 3 * 3 * 64], shB[4 * 3 * 3 * 64];
+  const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int q = blockIdx.y;
+  const int RT = (cout + 1) / 2, CT = (cin + 1) / 2, RB = (RT + 3) / 4;
+  const int rt0 = (blockIdx.z % RB) * 4, ct0 = (blockIdx.z / RB) * 4;
+  const bool hop = q >= 1 && q <= 8;
+  const size_t fsz = (size_t)Vh * 24 * Ls;
+  const int npts = Vh * Ls, gpp = (npts + 15) / 16;
+  // this block's 16-point groups
+  const int per = (2 * gpp + gridDim.x - 1) / gridDim.x;
+  const int first = blockIdx.x * per, last = min(first + per, 2 * gpp);
+  // row / column of this lane: channel, spin, part
+  const int ch = n >> 3, sp = (n >> 1) & 3, ri = n & 1;
+  const int a = 2 * (rt0 + wave) + ch, b = 2 * (ct0 + wave) + ch;
+  const bool rowt = rt0 + wave < RT, colt = ct0 + wave < CT;   // (wave-uniform)
+  const float sgn = ri ? 1.f : -1.f;   // re: u_r t_r - u_i t_i; im: u_r t_i + u_i t_r
+  flt4_t va[3], vb[3];
+  float edge[3], u[18];
+  const flt4_t zero = {0.f, 0.f, 0.f, 0.f};
+  const bool tail = (npts & 15) != 0;
+  // site and s of this lane's four points of a group; the lanes beyond the last point take
+  // the last ones, and their row operand is set to zero below.  (The division is that of
+  // the group's first point, in scalar registers.)
+  auto locate = [&](int grp, int& p, int& site, int& s) -> bool {
+    p = grp >= gpp ? 1 : 0;
+    const int P0 = (grp - p * gpp) * 16, base = P0 / Ls;
+    int r = P0 - base * Ls + 4 * g;
+    const bool ok = P0 + 4 * g < npts;
+    const int k = (r >= Ls) + (r >= 2 * Ls) + (r >= 3 * Ls);
+    site = ok ? base + k : Vh - 1;
+    s = ok ? r - k * Ls : Ls - 4;
+    return ok;
+  };
+  // rows and columns beyond the channels repeat the last one (their results are dropped)
+  const int ac = min(a, cout - 1), bc = min(b, cin - 1);
+  // the neighbour of group grp's site, fetched a group before the spinors it addresses
+  auto neighbour = [&](int grp) -> int {
+    int p, site, s;
+    locate(grp, p, site, s);
+    return (nbr + ((size_t)p * 8 + q - 1) * Vh)[(unsigned)site];
+  };
+  auto fetch = [&](int grp, int nb) {
+    int p, site, s;
+    const bool ok = locate(grp, p, site, s);
+    const unsigned comp = (unsigned)(ri + 6 * sp) * Ls + s, step = 2u * Ls;
+    if (rowt) {
+      const float* x = gr + ((size_t)ac * 2 + p) * fsz + (size_t)site * 24 * Ls + comp;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) va[c] = *reinterpret_cast<const flt4_t*>(x + c * step);
+      if (tail && !ok)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) va[c] = zero;
+    }
+    if (!colt) return;
+    const float* x = in + ((size_t)bc * 2 + (hop ? 1 - p : p)) * fsz +
+                     (size_t)(hop ? nb : site) * 24 * Ls + comp;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) vb[c] = *reinterpret_cast<const flt4_t*>(x + c * step);
+    if (hop) {
+#pragma unroll
+      for (int e = 0; e < 18; ++e) {
+        // scalar base and 32-bit offset (left alone, the compiler adds up 64-bit addresses)
+        typedef const __attribute__((address_space(1))) char* gptr_t;
+        gptr_t ub = (gptr_t)(links + (((size_t)p * 8 + q - 1) * 18 + e) * Vh);
+        asm("" : "+s"(ub));
+        u[e] = *(const __attribute__((address_space(1))) float*)(ub + 4u * (unsigned)site);
+      }
+    } else if (q == 9) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) edge[c] = s + 4 < Ls ? x[c * step + 4] : 0.f;
+    } else if (q == 10) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) edge[c] = s > 0 ? (x + c * step)[-1] : 0.f;
+    }
+  };
+  auto parts = [&](flt4_t v, unsigned (&hi)[2], unsigned (&mid)[2], unsigned (&lo)[2]) {
+    ptc_split_round(v[0], v[1], hi[0], mid[0], lo[0]);
+    ptc_split_round(v[2], v[3], hi[1], mid[1], lo[1]);
+  };
+  auto put = [](u32x2_t* d, const unsigned (&hi)[2], const unsigned (&mid)[2],
+                const unsigned (&lo)[2]) {
+    d[0] = u32x2_t{hi[0], hi[1]};
+    d[64] = u32x2_t{mid[0], mid[1]};
+    d[128] = u32x2_t{lo[0], lo[1]};
+  };
+  auto stage = [&]() {
+    unsigned hi[2], mid[2], lo[2];
+    if (rowt) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        parts(va[c], hi, mid, lo);
+        put(shA + (wave * 3 + c) * 192 + lane, hi, mid, lo);
+      }
+    }
+    if (colt) {
+      flt4_t x[3];
+      if (hop) {
+        // the other part of each component sits in the neighbouring lane
+        flt4_t o[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            o[c][i] = __uint_as_float(__builtin_amdgcn_update_dpp(
+                0, (int)__float_as_uint(vb[c][i]), 0xb1, 0xf, 0xf, true));   // quad_perm 1 0 3 2
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          x[c] = zero;
+#pragma unroll
+          for (int k = 0; k < 3; ++k) {
+            const float ur = u[2 * (k + 3 * c)], ui = sgn * u[2 * (k + 3 * c) + 1];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[c][i] = fmaf(ui, o[k][i], fmaf(ur, vb[k][i], x[c][i]));
+          }
+        }
+      } else if (q == 0) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) x[c] = vb[c];
+      } else if (q == 9) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) x[c] = flt4_t{vb[c][1], vb[c][2], vb[c][3], edge[c]};
+      } else {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) x[c] = flt4_t{edge[c], vb[c][0], vb[c][1], vb[c][2]};
+      }
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        parts(x[c], hi, mid, lo);
+        put(shB + (wave * 3 + c) * 192 + lane, hi, mid, lo);
+      }
+    }
+  };
+  const int tr = 2 * (wave >> 1), tc = 2 * (wave & 1);   // this wave's quadrant
+  double acc[2][2][4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.0;
+  int nb = 0;
+  if (first < last) {
+    if (hop) nb = neighbour(first);
+    fetch(first, nb);
+    if (hop && first + 1 < last) nb = neighbour(first + 1);
+  }
+  for (int grp = first; grp < last; ++grp) {
+    stage();
+    __syncthreads();
+    if (grp + 1 < last) {
+      fetch(grp + 1, nb);
+      if (hop && grp + 2 < last) nb = neighbour(grp + 2);
+    }
+    if (rt0 + tr < RT && ct0 + tc < CT) {
+      flt4_t d[2][2] = {{zero, zero}, {zero, zero}};
+      // parts (a0 a1) of the row tiles times (b0 b1) of the column tiles; 0 hi, 1 mid, 2 lo
+      auto mma = [&](int c, int a0, int a1, int b0, int b1) {
+        b8_t A[2], B[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const u32x2_t* x = shA + ((tr + i) * 3 + c) * 192 + lane;
+          const u32x2_t* y = shB + ((tc + i) * 3 + c) * 192 + lane;
+          const u32x2_t x0 = x[64 * a0], x1 = x[64 * a1], y0 = y[64 * b0], y1 = y[64 * b1];
+          A[i] = __builtin_bit_cast(b8_t, u32x4_t{x0[0], x0[1], x1[0], x1[1]});
+          B[i] = __builtin_bit_cast(b8_t, u32x4_t{y0[0], y0[1], y1[0], y1[1]});
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            d[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[i], B[j], d[i][j], 0, 0, 0);
+      };
+      // the small products of all three colours first: only the three large ones round at
+      // the size of the result
+#pragma unroll
+      for (int c = 0; c < 3; ++c) mma(c, 0, 2, 2, 0);
+      // (parts read anew for each pass come as whole operands; kept, they cost moves)
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int c = 0; c < 3; ++c) mma(c, 1, 0, 0, 1);
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int c = 0; c < 3; ++c) mma(c, 1, 0, 1, 0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[i][j][r] += (double)d[i][j][r];
+    }
+    __syncthreads();
+  }
+  // P -> g conj(t): the lane of t_re holds (g_re, g_im) t_re in registers 2 k, 2 k + 1, its
+  // neighbour those of t_im;  re = g_re t_re + g_im t_im,  im = g_im t_re - g_re t_im
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int ga = 2 * (rt0 + tr + i) + (g >> 1), gb = 2 * (ct0 + tc + j) + ch;
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const double x = acc[i][j][2 * k], py = __shfl_xor(acc[i][j][2 * k + 1], 1, 64);
+        const double v = ri ? py - x : x + py;
+        const int al = 2 * (g & 1) + k;
+        if (ga < cout && gb < cin)
+          partial[(((size_t)(q * cin + gb) * cout + ga) * gridDim.x + blockIdx.x) * 32 +
+                  2 * (al * 4 + sp) + ri] = v;
+      }
+    }
+}
+
 // out[(y z) 32 + k] = sum over the nblk block partials, fixed order
 __global__ void __launch_bounds__(64)
 k_ptc_wgrad_finish(double* __restrict__ out, const double* __restrict__ partial, int nblk,
@@ -630,10 +885,28 @@ hipError_t launch_ptc_layer(bool adj, float* out, const float* in, int cin, int 
   return hipGetLastError();
 }
 
-hipError_t launch_ptc_wgrad(double* G, double* partial, int nblk, const float* g, const float* in,
+hipError_t launch_ptc_wgrad(double* G, double* partial, int maxblk, const float* g, const float* in,
                             int cin, int cout, const float* links, const int* nbr, int Vh, int Ls,
                             hipStream_t st) {
   if (cout < 1) return hipErrorInvalidValue;
+  const int nyz = kPtcPaths * cin * cout;
+  const size_t pts = (size_t)2 * Vh * Ls;
+  // The matrix-core form needs four consecutive s per lane.  Its time hardly depends on how
+  // far its 8 x 8 channel tiles are filled (8^3 x 16, Ls = 16: 8 -> 8 507 us, 1 -> 8 377),
+  // the other one's is that of cin cout (1290 and 181): they would be equal near 25 products
+  // a tile group, and the line lies a little above.
+  const int tb = ((cout + 1) / 2 + 3) / 4 * (((cin + 1) / 2 + 3) / 4);
+  if (Ls % 4 == 0 && cin * cout > 32 * tb) {
+    // four 16-point groups a block until all maxblk blocks are there (with the 64 groups
+    // that the other form takes, 8 -> 8 at 4^3 x 8, Ls = 8, had 44 blocks on 256 CUs)
+    const int nblk = (int)std::max<size_t>(1, std::min<size_t>(maxblk, pts / 64));
+    hipLaunchKernelGGL(k_ptc_wgrad_mfma, dim3(nblk, kPtcPaths, tb), dim3(256), 0, st, partial, g,
+                       in, cin, cout, links, nbr, Vh, Ls);
+    hipLaunchKernelGGL(k_ptc_wgrad_finish, dim3(nyz), dim3(64), 0, st, G, partial, nblk, nyz);
+    return hipGetLastError();
+  }
+  // about 1024 points per block
+  const int nblk = (int)std::max<size_t>(1, std::min<size_t>(maxblk, pts / 1024));
   // two output channels per thread: four need 128 accumulators (266 registers,
   // one wave per SIMD), which is slower
   const int ag = cout % 2 == 0 ? 2 : 1;
@@ -644,7 +917,6 @@ hipError_t launch_ptc_wgrad(double* G, double* partial, int nblk, const float* g
   else
     hipLaunchKernelGGL(k_ptc_wgrad<1>, grid, dim3(256), 0, st, partial, g, in, cin, cout, links,
                        nbr, Vh, Ls);
-  const int nyz = kPtcPaths * cin * cout;
   hipLaunchKernelGGL(k_ptc_wgrad_finish, dim3(nyz), dim3(64), 0, st, G, partial, nblk, nyz);
   return hipGetLastError();
 }
