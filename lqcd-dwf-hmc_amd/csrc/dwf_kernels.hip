@@ -1252,22 +1252,31 @@ static hipError_t launch_combo(int op, bool mat, bool addx, bool out2, dim3 g, d
 static void finish_norm(const double* partial, unsigned nblocks, double* result, hipStream_t st,
                         double* host);
 
+// Block of k_dwf: compiled Ls (lsc) or runtime Ls, sites, threads, LDS.
+struct DwfShape {
+  bool lsc = false;
+  int spb = 0;
+  unsigned threads = 0;
+  size_t lds = 0;
+};
+
+// The forms that the operator launches take, and the block of k_dwf for them.  Both
+// operator kernels go by this rule, so what is accepted does not depend on the volume.
 template <typename T>
-static hipError_t launch_dwf_t(int op, void* out, const void* in, const void* links,
-                               const int* nbr, int parity, int Vh, int Ls, const Epi& e,
-                               hipStream_t st, unsigned* nblocks) {
+static hipError_t dwf_shape_t(int op, const void* out, int Ls, const Epi& e, DwfShape* shape) {
   using C = typename St<T>::C;
   const bool mat = e.E != nullptr;
   const bool addx = e.X != nullptr;
   const bool out2 = e.out2 != nullptr;
-  if (out2 && !mat) return hipErrorInvalidValue;
-  if (e.nrm_partial && !mat) return hipErrorInvalidValue;
+  if (!mat && (op != K_HOP || addx || out2 || e.nrm_partial)) return hipErrorInvalidValue;
+  if (op == K_SITE && addx && !out2) return hipErrorInvalidValue;
+  if (op == K_HOPDAG && out2 && !addx) return hipErrorInvalidValue;
+  if ((e.G && !addx) || (e.X2 && !out2)) return hipErrorInvalidValue;
   const int vec = KCfg<T>::VEC;
-  const bool lsc = (Ls == 4 || Ls == 8 || Ls == 12 || Ls == 16) && Ls % vec == 0;
-  int spb = lsc ? spb_of<T>(Ls, vec) : KCfg<T>::THREADS / Ls;
+  shape->lsc = (Ls == 4 || Ls == 8 || Ls == 12 || Ls == 16) && Ls % vec == 0;
+  int spb = shape->lsc ? spb_of<T>(Ls, vec) : KCfg<T>::THREADS / Ls;
   if (spb < 1) return hipErrorInvalidValue;
   const size_t cs = sizeof(C);
-  if ((e.G && (!mat || !addx)) || (e.X2 && !out2)) return hipErrorInvalidValue;
   const size_t matb =
       mat ? 2 * (size_t)Ls * Ls * cs * (1 + (out2 ? 1 : 0) + (e.G ? 1 : 0)) : 0;
   const size_t lds_cap = 64 * 1024;
@@ -1275,55 +1284,74 @@ static hipError_t launch_dwf_t(int op, void* out, const void* in, const void* li
     const bool pk = std::is_same<T, __half>::value && KCfg<T>::VEC == 2 && mfma_ls(Ls) &&
                     DWF_HOP_PK16;
     const size_t stage = (op == K_SITE) ? 0 : (size_t)((pk ? kPkStride : 144) + 8) * sp * cs;
-    const size_t epi = mat ? (size_t)sp * (mfma_ls(Ls) && lsc ? 12 * 17 : 2 * (12 * Ls + 1)) * cs : 0;
+    const size_t epi = mat ? (size_t)sp * (mfma_ls(Ls) && shape->lsc ? 12 * 17 : 2 * (12 * Ls + 1)) * cs : 0;
     return (stage > epi ? stage : epi) + matb;
   };
   // The compiled-Ls kernels fix their block at THREADS / (Ls / VEC) sites; when
   // that block's link staging exceeds the LDS cap (FP64 and FP32 at Ls = 4) the
-  // runtime-Ls kernel below runs instead, with fewer sites per block.
+  // runtime-Ls kernel runs instead, with fewer sites per block.
   // the fused CG updates, and an output that is not stored, exist in the
   // matrix-core epilogue only
-  const bool mfma_path = mat && mfma_ls(Ls) && lsc && lds_for(spb) <= lds_cap;
+  const bool mfma_path = mat && mfma_ls(Ls) && shape->lsc && lds_for(spb) <= lds_cap;
   if (e.upd && !(mfma_path && (op == K_SITE ? addx : !out2))) return hipErrorInvalidValue;
   if (!out && !e.upd && !(mfma_path && out2)) return hipErrorInvalidValue;
-  const int VhV = Vh << e.nrs;   // virtual sites (site, rhs)
-  if (lsc && lds_for(spb) <= lds_cap) {
-    const size_t lds = lds_for(spb);
-    const dim3 block(spb * tps_of<T>(Ls, vec)), grid((VhV + spb - 1) / spb);
-    if (e.fin_partial && block.x % 64) return hipErrorInvalidValue;   // block_sum: whole waves
-    *nblocks = grid.x;
-    switch (Ls) {
-      case 4: return launch_combo<T, 4>(op, mat, addx, out2, grid, block, lds, st, out, in, links, nbr, parity, Vh, Ls, spb, e);
-      case 8: return launch_combo<T, 8>(op, mat, addx, out2, grid, block, lds, st, out, in, links, nbr, parity, Vh, Ls, spb, e);
-      case 12: return launch_combo<T, 12>(op, mat, addx, out2, grid, block, lds, st, out, in, links, nbr, parity, Vh, Ls, spb, e);
-      case 16: return launch_combo<T, 16>(op, mat, addx, out2, grid, block, lds, st, out, in, links, nbr, parity, Vh, Ls, spb, e);
-      default: break;
-    }
+  if (shape->lsc && lds_for(spb) <= lds_cap) {
+    shape->threads = spb * tps_of<T>(Ls, vec);
+  } else {
+    shape->lsc = false;
+    spb = KCfg<T>::THREADS / Ls;
+    while (spb > 1 && lds_for(spb) > lds_cap) --spb;
+    if (lds_for(spb) > lds_cap) return hipErrorInvalidValue;
+    shape->threads = spb * Ls;
   }
-  spb = KCfg<T>::THREADS / Ls;
-  while (spb > 1 && lds_for(spb) > lds_cap) --spb;
-  if (lds_for(spb) > lds_cap) return hipErrorInvalidValue;
-  const size_t lds = lds_for(spb);
-  const dim3 block(spb * Ls), grid((VhV + spb - 1) / spb);
-  if (e.fin_partial && block.x % 64) return hipErrorInvalidValue;
+  if (e.fin_partial && shape->threads % 64) return hipErrorInvalidValue;   // block_sum: whole waves
+  shape->spb = spb;
+  shape->lds = lds_for(spb);
+  return hipSuccess;
+}
+
+template <typename T>
+static hipError_t launch_dwf_t(const DwfShape& sh, int op, void* out, const void* in,
+                               const void* links, const int* nbr, int parity, int Vh, int Ls,
+                               const Epi& e, hipStream_t st, unsigned* nblocks) {
+  const bool mat = e.E != nullptr, addx = e.X != nullptr, out2 = e.out2 != nullptr;
+  const int VhV = Vh << e.nrs;   // virtual sites (site, rhs)
+  const dim3 block(sh.threads), grid((VhV + sh.spb - 1) / sh.spb);
   *nblocks = grid.x;
-  return launch_combo<T, 0>(op, mat, addx, out2, grid, block, lds, st, out, in, links, nbr,
-                            parity, Vh, Ls, spb, e);
+#define LC(L)                                                                                   \
+  return launch_combo<T, L>(op, mat, addx, out2, grid, block, sh.lds, st, out, in, links, nbr,  \
+                            parity, Vh, Ls, sh.spb, e)
+  if (!sh.lsc) LC(0);
+  switch (Ls) {
+    case 4: LC(4);
+    case 8: LC(8);
+    case 12: LC(12);
+    default: LC(16);
+  }
+#undef LC
 }
 
 hipError_t launch_dwf(int prec, int op, void* out, const void* in, const void* links,
                       const int* nbr, int parity, int Vh, int Ls, const Epi& e,
                       hipStream_t st) {
+  DwfShape sh;
   hipError_t err = hipErrorInvalidValue;
+  switch (prec) {
+    case P64: err = dwf_shape_t<double>(op, out, Ls, e, &sh); break;
+    case P32: err = dwf_shape_t<float>(op, out, Ls, e, &sh); break;
+    case P16: err = dwf_shape_t<__half>(op, out, Ls, e, &sh); break;
+    case PBF16: err = dwf_shape_t<__hip_bfloat16>(op, out, Ls, e, &sh); break;
+  }
+  if (err != hipSuccess) return err;
   unsigned nb = 0;
   if (small_dwf_applies(prec, op, Vh, Ls, e))
     err = launch_dwf_small(prec, op, out, in, links, nbr, parity, Vh, Ls, e, st, &nb);
   else switch (prec) {
-    case P64: err = launch_dwf_t<double>(op, out, in, links, nbr, parity, Vh, Ls, e, st, &nb); break;
-    case P32: err = launch_dwf_t<float>(op, out, in, links, nbr, parity, Vh, Ls, e, st, &nb); break;
-    case P16: err = launch_dwf_t<__half>(op, out, in, links, nbr, parity, Vh, Ls, e, st, &nb); break;
-    case PBF16:
-      err = launch_dwf_t<__hip_bfloat16>(op, out, in, links, nbr, parity, Vh, Ls, e, st, &nb);
+    case P64: err = launch_dwf_t<double>(sh, op, out, in, links, nbr, parity, Vh, Ls, e, st, &nb); break;
+    case P32: err = launch_dwf_t<float>(sh, op, out, in, links, nbr, parity, Vh, Ls, e, st, &nb); break;
+    case P16: err = launch_dwf_t<__half>(sh, op, out, in, links, nbr, parity, Vh, Ls, e, st, &nb); break;
+    default:
+      err = launch_dwf_t<__hip_bfloat16>(sh, op, out, in, links, nbr, parity, Vh, Ls, e, st, &nb);
       break;
   }
   if (e.nblocks_out) *e.nblocks_out = nb;

@@ -329,11 +329,6 @@ static hipError_t launch_small_t(int op, void* out, const void* in, const void* 
 hipError_t launch_dwf_small(int prec, int op, void* out, const void* in, const void* links,
                             const int* nbr, int parity, int Vh, int Ls, const Epi& e,
                             hipStream_t st, unsigned* nblocks) {
-  // the combinations that k_dwf refuses
-  const bool mat = e.E != nullptr, addx = e.X != nullptr, out2 = e.out2 != nullptr;
-  if ((!mat && (op != K_HOP || addx || out2 || e.nrm_partial)) || (e.G && !addx) ||
-      (e.X2 && !out2) || (e.upd && !(op == K_SITE ? addx : !out2)) || (!out && !e.upd && !out2))
-    return hipErrorInvalidValue;
   const size_t lds = small_lds(prec, op, Ls, e);
   switch (prec) {
     case P64: return launch_small_t<double>(op, out, in, links, nbr, parity, Vh, Ls, e, lds, st, nblocks);
