@@ -73,7 +73,7 @@ k_dwf_small(const SmallArgs<T> a) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int NS = 64 / Ls, ls = lane / Ls, s = lane - ls * Ls;
-  const int blk = blockIdx.x;
+  const int blk = xcd_block(blockIdx.x, gridDim.x);
   const int v = blk * NS + ls;                     // virtual site (site * nr + rhs)
   const bool valid = ls < NS && v < (a.Vh << a.nrs);
   const int site = valid ? v >> a.nrs : 0;
@@ -277,27 +277,49 @@ static size_t small_lds(int prec, int op, int Ls, const Epi& e) {
   return ((op == K_SITE ? 48 : 96) * 64 + mats) * (prec == P64 ? 8 : 4);
 }
 
-// The line between this kernel and k_dwf, in blocks of this one (64 / Ls sites), from
-// D^+D times of both over volumes of 512 to 442,000 sites and Ls = 4 to 22 (us, k_dwf
-// against this kernel):
-// * Ls = 12, 16, where k_dwf has the matrix cores: 410 blocks 58-86 against 40-58, 615
-//   61-88 / 53-81, 820 61-91 / 66-98; BF16, whose k_dwf hop is not packed, 768 72 / 50,
-//   2000 101 / 96.
-// * Ls = 8 (compiled, no matrix cores): 1000 73-110 / 59-90, 2048 85-163 / 93-152; 16-bit
-//   8192 338 / 284, 27648 887 / 944.
-// * other Ls, and Ls = 4, where k_dwf has a runtime Ls or two-byte accesses: up to Ls = 10
-//   FP64 1334 166 / 122, 5462 461 / 441, 36864 2714 / 2778, the others at every size
-//   (Ls = 10, 36864: FP32 1908 / 1657, FP16 1870 / 1426); beyond, FP64 and FP32 1250
-//   104-152 / 78-121, 2000 110-162 / 107-172, 16-bit 8192 382 / 323, 16384 638 / 605.
+// The line between this kernel and k_dwf, in blocks of this one (64 / Ls sites): up to it
+// this kernel was the faster or within a few per cent of it (but for single sizes: site FP16
+// Ls = 9 2963 11.2 / 13.0, where it is ahead below and above).  Measured over volumes of 256
+// to 663,000 sites for every Ls below, per launch (us, k_dwf against this kernel, blocks):
+// * Ls = 12, 16, where k_dwf has the matrix cores: hop FP64 Ls = 16 512 14.4 / 10.8,
+//   1024 15.1 / 19.4; BF16, whose k_dwf hop is not packed, 1024 14.5 / 9.9, 1800 14.8 / 16.9.
+// * Ls = 8 (compiled, no matrix cores): hop FP64 900 19.5 / 17.9, 1728
+//   26.9 / 28.6; FP16 8192 72 / 52; site FP16 900 5.7 / 5.2, 8192 16.6 / 26.1.
+// * Ls up to 11 otherwise, where k_dwf has a runtime Ls (one element per access), ahead at
+//   most sizes: hop FP32 Ls = 10 36864 356 / 332, site FP16 Ls = 6 33178 180 / 105; not
+//   so FP64 hops that fill the GPU (Ls = 6 9831 155 / 171), nor FP16 sites at Ls = 10
+//   (5462 14.2 / 21.1).
+// * larger Ls: the transposed matrices take LDS, and from Ls = 17 on lanes idle: FP16 site
+//   Ls = 14 1024 7.3 / 6.5, 3456 10.9 / 16.1; hop FP16 Ls = 22 2048 28 / 20, 6912 47 / 58.
+// A hop without E lacks the epilogue that this kernel spreads over its waves, and a site
+// launch the gathers: both leave it earlier than a hop does.
+static long small_max_blocks(int prec, int op, bool mat, int Ls) {
+  constexpr long all = 1L << 40;
+  const bool f64 = prec == P64, f32 = prec == P32, b16 = !f64 && !f32;
+  if (op == K_SITE) {
+    if (Ls == 4) return f64 ? 600 : f32 ? 1000 : all;
+    if (Ls == 8) return f64 ? 600 : f32 ? 900 : 1200;
+    if (Ls == 10) return b16 ? 2000 : all;
+    if (Ls == 12) return b16 ? 1000 : 400;
+    if (Ls == 16) return f64 ? 250 : 400;
+    return Ls <= 11 ? all : f64 ? 1500 : 1100;
+  }
+  if (Ls == 12 || Ls == 16) return prec == PBF16 ? 1500 : 640;
+  if (Ls == 8) return b16 ? 8192 : mat ? 1300 : f64 ? 700 : 1000;
+  if (Ls <= 5 || (Ls <= 7 && !f64)) return all;
+  if (Ls <= 10) {
+    if (f64) return !mat ? 1500 : Ls == 9 ? 2000 : 7000;
+    if (f32) return !mat || Ls == 9 ? 20000 : all;
+    return mat ? all : 40000;
+  }
+  if (b16) return Ls < 20 || (mat && Ls < 22) ? 8192 : 2400;
+  return mat ? (f64 ? 1200 : 1500) : f64 ? 700 : 1000;
+}
 bool small_dwf_applies(int prec, int op, int Vh, int Ls, const Epi& e) {
   if (Ls > 22 || small_lds(prec, op, Ls, e) > 64 * 1024 - 256) return false;
   const int NS = 64 / Ls;
   const long blocks = (((long)Vh << e.nrs) + NS - 1) / NS;
-  const bool b16 = prec != P64 && prec != P32;
-  if (Ls == 12 || Ls == 16) return blocks <= (prec == PBF16 ? 1500 : 640);
-  if (Ls == 8) return blocks <= (b16 ? 8192 : 1300);
-  if (Ls <= 10) return prec != P64 || blocks <= 10000;
-  return blocks <= (b16 ? 8192 : 1500);
+  return blocks <= small_max_blocks(prec, op, e.E != nullptr, Ls);
 }
 
 template <typename T>

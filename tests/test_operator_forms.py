@@ -1,6 +1,9 @@
-"""What the operator launch accepts does not depend on the volume: the forms that k_dwf
-refuses are refused on a small lattice too, where k_dwf_small would run.  No form below
-reaches a kernel, so the pointers are never read."""
+"""Host-side rules of the operator launch (nothing here reaches a kernel, so the pointers
+are never read).
+
+What it accepts does not depend on the volume: the forms that k_dwf refuses are refused on a
+small lattice too, where k_dwf_small would run.  And which of the two kernels a launch takes
+follows what either one was measured to take."""
 import os
 import shutil
 import subprocess
@@ -8,7 +11,7 @@ import subprocess
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB = os.path.join(ROOT, "lqcd-dwf-hmc_amd", "dwf_amd")
 
-SOURCE = r"""
+FORMS = r"""
 #include <cstdio>
 #include "dwf_kernels.h"
 using namespace dwf;
@@ -50,12 +53,53 @@ int main() {
 """
 
 
-def test_refused_on_every_volume(tmp_path):
-    src, exe = tmp_path / "forms.hip", str(tmp_path / "forms")
-    src.write_text(SOURCE)
+# precision, Ls, blocks of 64 / Ls sites, kind, us of k_dwf, us of k_dwf_small
+MEASURED = """
+P64 16 512 hop 14.4 10.8      P64 16 1024 hop 15.1 19.4     PBF16 16 1024 hop 14.5 9.9
+P64 8 900 hop 19.5 17.9       P16 8 8192 hop 72.4 51.6      P16 8 8192 site 16.6 26.1
+P32 10 36864 hop 355.6 331.9  P16 6 33178 site 179.9 105.2  P64 6 9831 hop 155.1 171.0
+P16 10 5462 site 14.2 21.1    P16 14 1024 site 7.3 6.5      P16 14 3456 site 10.9 16.1
+P16 22 2048 hop 28.1 20.4     P16 22 6912 hop 47.1 58.4     P16 20 6912 scalar 29.3 35.3
+P64 9 2963 scalar 36.8 47.0   P32 4 4096 site 11.9 15.9     P64 4 2560 site 11.0 13.4
+PBF16 16 1024 site 5.0 6.7    P16 22 3600 scalar 19.5 22.5  P16 4 4096 site 15.9 14.7
+"""
+
+RULE = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "dwf_kernels.h"
+using namespace dwf;
+int main(int, char** argv) {   // precision, Ls, Vh, operation, with E
+  static double mem[1];
+  Epi e;
+  if (std::atoi(argv[5])) e.E = mem;
+  std::printf("%d", (int)small_dwf_applies(std::atoi(argv[1]), std::atoi(argv[4]),
+                                           std::atoi(argv[3]), std::atoi(argv[2]), e));
+}
+"""
+
+
+def compiled(tmp_path, source):
+    src, exe = tmp_path / "probe.hip", str(tmp_path / "probe")
+    src.write_text(source)
     hipcc = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
     subprocess.run([hipcc, "--offload-arch=gfx950", "-std=c++17", "-I",
                     os.path.join(ROOT, "lqcd-dwf-hmc_amd", "csrc"), str(src), "-L", LIB, "-ldwfhip",
                     f"-Wl,-rpath,{LIB}", "-o", exe], check=True)
-    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    return exe
+
+
+def test_refused_on_every_volume(tmp_path):
+    r = subprocess.run([compiled(tmp_path, FORMS)], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
+
+
+def test_kernel_of_a_launch(tmp_path):
+    exe = compiled(tmp_path, RULE)
+    words = MEASURED.split()
+    for prec, Ls, blocks, kind, full, small in zip(*[iter(words)] * 6):
+        p = ("P64", "P32", "P16", "PBF16").index(prec)
+        Vh = int(blocks) * (64 // int(Ls))
+        args = [p, Ls, Vh, 0 if kind == "site" else 1, 0 if kind == "scalar" else 1]
+        r = subprocess.run([exe, *map(str, args)], capture_output=True, text=True, timeout=60)
+        assert r.stdout == ("1" if float(small) < float(full) else "0"), (prec, Ls, blocks, kind)
