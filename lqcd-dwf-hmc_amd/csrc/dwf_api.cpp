@@ -15,6 +15,7 @@
 #include <cstdint>
 #include <cmath>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <utility>
@@ -281,6 +282,7 @@ struct dwf_fopr_s {
   bool have_config = false;
   std::vector<ChiMat> hmats;   // host copies of the matrices (long double)
   double* hop_partial = nullptr;   // block partials of fused norms (Vh doubles)
+  int kernel = 0;                  // Epi::kernel of its launches
 };
 
 static size_t cbytes(int prec) { return prec == P64 ? 8 : 4; }
@@ -440,6 +442,12 @@ static int get_work(dwf_fopr_s* op, int i, void** out) {
 }
 
 // launch helpers ------------------------------------------------------------
+static hipError_t launch_op(dwf_fopr_s* op, int kop, void* out, const void* in, int parity,
+                            Epi& e) {
+  e.kernel = op->kernel;
+  return launch_dwf(op->prec, kop, out, in, op->links, op->nbr, parity, op->Vh, op->Ls, e,
+                    g_ctx.stream);
+}
 static int run_site(dwf_fopr_s* op, void* out, const void* in, int mid, void* out2 = nullptr,
                     int fid = -1) {
   Epi e;
@@ -448,8 +456,7 @@ static int run_site(dwf_fopr_s* op, void* out, const void* in, int mid, void* ou
     e.out2 = out2;
     e.F = mat(op, fid);
   }
-  HIPCHK(launch_dwf(op->prec, K_SITE, out, in, op->links, op->nbr, 0, op->Vh, op->Ls, e,
-                    g_ctx.stream));
+  HIPCHK(launch_op(op, K_SITE, out, in, 0, e));
   return DWF_OK;
 }
 static int run_hop(dwf_fopr_s* op, bool dag, int parity, void* out, const void* in, int mid,
@@ -463,8 +470,7 @@ static int run_hop(dwf_fopr_s* op, bool dag, int parity, void* out, const void* 
     e.out2 = out2;
     e.F = mat(op, fid);
   }
-  HIPCHK(launch_dwf(op->prec, dag ? K_HOPDAG : K_HOP, out, in, op->links, op->nbr, parity,
-                    op->Vh, op->Ls, e, g_ctx.stream));
+  HIPCHK(launch_op(op, dag ? K_HOPDAG : K_HOP, out, in, parity, e));
   return DWF_OK;
 }
 
@@ -515,8 +521,7 @@ static int op_Ddag_u2(dwf_fopr_s* op, void* v, const void* u2) {
   g.E = mat(op, M_G2);
   g.X = u2;
   g.G = mat(op, M_DEET);
-  HIPCHK(launch_dwf(op->prec, K_HOPDAG, v, t1, op->links, op->nbr, 0, op->Vh, op->Ls, g,
-                    g_ctx.stream));
+  HIPCHK(launch_op(op, K_HOPDAG, v, t1, 0, g));
   return DWF_OK;
 }
 static int op_DdagD(dwf_fopr_s* op, void* v, const void* w) {
@@ -559,8 +564,7 @@ static int op_DdagD_nrm(dwf_fopr_s* op, void* v, const void* w, double* nrm,
   e.nrm_partial = op->hop_partial;
   e.nrm_result = nrm;
   const bool keep_u = !u_unstored(op);
-  HIPCHK(launch_dwf(op->prec, K_HOP, keep_u ? u : nullptr, t1, op->links, op->nbr, 0, op->Vh,
-                    op->Ls, e, g_ctx.stream));
+  HIPCHK(launch_op(op, K_HOP, keep_u ? u : nullptr, t1, 0, e));
   return keep_u ? op_Ddag(op, v, u, u2) : op_Ddag_u2(op, v, u2);
 }
 // One CG step's operator part with the residual update fused into the last
@@ -589,16 +593,14 @@ static int op_DdagD_cg(dwf_fopr_s* op, const void* p, const void* mpw, double* p
   unsigned nb2 = 0;
   e.nrm_defer = true;   // added up by the last block of the next hop
   e.nblocks_out = &nb2;
-  HIPCHK(launch_dwf(op->prec, K_HOP, nullptr, t1, op->links, op->nbr, 0, op->Vh, op->Ls, e,
-                    g_ctx.stream));
+  HIPCHK(launch_op(op, K_HOP, nullptr, t1, 0, e));
   {
     Epi h;   // first hop of D^dag; its last block adds up |D p|^2
     h.E = mat(op, M_G1);
     h.fin_partial = op->hop_partial;
     h.fin_n = nb2;
     h.fin_result = pap;
-    HIPCHK(launch_dwf(op->prec, K_HOPDAG, t1, u2, op->links, op->nbr, 1, op->Vh, op->Ls, h,
-                      g_ctx.stream));
+    HIPCHK(launch_op(op, K_HOPDAG, t1, u2, 1, h));
   }
   Epi g;
   g.E = mat(op, M_G2);
@@ -610,8 +612,7 @@ static int op_DdagD_cg(dwf_fopr_s* op, const void* p, const void* mpw, double* p
   g.nrm_partial = op->hop_partial;
   g.nrm_result = rr_new;
   g.nrm_host = rr_host;
-  HIPCHK(launch_dwf(op->prec, K_HOPDAG, nullptr, t1, op->links, op->nbr, 0, op->Vh, op->Ls, g,
-                    g_ctx.stream));
+  HIPCHK(launch_op(op, K_HOPDAG, nullptr, t1, 0, g));
   return DWF_OK;
 }
 static int op_DDdag(dwf_fopr_s* op, void* v, const void* w) {
@@ -648,8 +649,7 @@ static int op_Deo(dwf_fopr_s* op, void* v, const void* w, int parity) {
   if (op->deo_is_scalar) {
     Epi e;
     e.scale = op->deo_scale;
-    HIPCHK(launch_dwf(op->prec, K_HOP, v, src, op->links, op->nbr, parity, op->Vh, op->Ls, e,
-                      g_ctx.stream));
+    HIPCHK(launch_op(op, K_HOP, v, src, parity, e));
     return DWF_OK;
   }
   RC(run_hop(op, false, parity, v, src, M_DEO));
@@ -750,6 +750,10 @@ int dwf_fopr_create(const dwf_fopr_params* p, dwf_fopr* out) {
     op->c[s] = p->coefficient_c ? p->coefficient_c[s] : p->c_uniform;
   }
   op->nelem = (size_t)op->Vh * 24 * Ls;
+  // which operator kernel its launches take where both could (the tests run either one)
+  const char* kernel = std::getenv("DWF_HOP_KERNEL");
+  if (kernel && !std::strcmp(kernel, "small")) op->kernel = EPI_SMALL;
+  if (kernel && !std::strcmp(kernel, "full")) op->kernel = EPI_FULL;
   auto cleanup = [&](int rc) {
     dwf_fopr_destroy(op);
     return rc;
@@ -1063,8 +1067,7 @@ static int site_m(dwf_fopr op, void* out, const void* in, const void* E, void* o
   e.E = E;
   e.out2 = out2;
   e.F = F;
-  HIPCHK(launch_dwf(op->prec, K_SITE, out, in, op->links, op->nbr, 0, op->Vh, op->Ls, e,
-                    g_ctx.stream));
+  HIPCHK(launch_op(op, K_SITE, out, in, 0, e));
   return DWF_OK;
 }
 
@@ -1090,8 +1093,7 @@ static int lpc_apply_K(dwf_lpc_s* p, void* v, const void* w) {
     e.out2 = v;
     e.F = lpc_mat(p, 1 + k);
     e.X2 = v;
-    HIPCHK(launch_dwf(op->prec, K_HOP, k < L ? zh : tmp, t1, op->links, op->nbr, 0, op->Vh,
-                      op->Ls, e, g_ctx.stream));
+    HIPCHK(launch_op(op, K_HOP, k < L ? zh : tmp, t1, 0, e));
     zin = zh;
   }
   return DWF_OK;
@@ -1116,8 +1118,7 @@ static int lpc_apply_Kdag(dwf_lpc_s* p, void* v, const void* w) {
       e.out2 = th;
       e.F = mat(op, M_DIT);
     }
-    HIPCHK(launch_dwf(op->prec, K_HOPDAG, k > 0 ? tmp : v, t1, op->links, op->nbr, 0, op->Vh,
-                      op->Ls, e, g_ctx.stream));
+    HIPCHK(launch_op(op, K_HOPDAG, k > 0 ? tmp : v, t1, 0, e));
   }
   return DWF_OK;
 }
@@ -1320,7 +1321,7 @@ struct FastCG {
       e.upd = x;
       e.unum = res + cur;
       e.uden = res + PAP;
-      HIPCHK(launch_dwf(op->prec, K_SITE, p2, r, op->links, op->nbr, 0, op->Vh, op->Ls, e, st));
+      HIPCHK(launch_op(op, K_SITE, p2, r, 0, e));
       std::swap(p, p2);
     } else {
       RC(op_DdagD_nrm(op, q, p, res + PAP, pre ? q : nullptr));
@@ -1333,8 +1334,7 @@ struct FastCG {
         e.xden = res + cur;
         e.out2 = q;
         e.F = mat(op, M_PRE);
-        HIPCHK(launch_dwf(op->prec, K_SITE, p2, r, op->links, op->nbr, 0, op->Vh, op->Ls, e,
-                          st));
+        HIPCHK(launch_op(op, K_SITE, p2, r, 0, e));
         std::swap(p, p2);
       } else {
         HIPCHK(launch_aypx_dev(pr, p, r, res + nxt, res + cur, n, st));
@@ -2199,6 +2199,7 @@ static void ms_build_stages(dwf_msbatch_s* m) {
       G.links = M.op->links;
       G.nbr = M.op->nbr;
       G.Vh = M.op->Vh;
+      G.e.kernel = M.op->kernel;
       G.e.nrs = M.nrs;
       G.e.rstride = M.op->nelem;
       fill(M, G);

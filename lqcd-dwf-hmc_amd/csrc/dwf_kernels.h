@@ -64,7 +64,9 @@ struct Epi {
   // their spinors of one 4D site share the staged links (Vh stays the 4D count)
   int nrs = 0;
   size_t rstride = 0;
+  int kernel = 0;   // EPI_SMALL, EPI_FULL: that kernel where it can run; 0: by the rule
 };
+enum EpiKernel { EPI_SMALL = 1, EPI_FULL = 2 };
 
 // The same launch by the small-lattice kernel (dwf_small.hip), and the rule for it.
 bool small_dwf_applies(int prec, int op, int Vh, int Ls, const Epi& e);

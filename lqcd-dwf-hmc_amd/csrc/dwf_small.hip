@@ -317,6 +317,7 @@ static long small_max_blocks(int prec, int op, bool mat, int Ls) {
 }
 bool small_dwf_applies(int prec, int op, int Vh, int Ls, const Epi& e) {
   if (Ls > 22 || small_lds(prec, op, Ls, e) > 64 * 1024 - 256) return false;
+  if (e.kernel) return e.kernel == EPI_SMALL;
   const int NS = 64 / Ls;
   const long blocks = (((long)Vh << e.nrs) + NS - 1) / NS;
   return blocks <= small_max_blocks(prec, op, e.E != nullptr, Ls);

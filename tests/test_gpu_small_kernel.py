@@ -1,8 +1,8 @@
 """The small-lattice operator kernel and k_dwf on both sides of the rule between them.
 
 The rule counts blocks of 64 / Ls sites; the lattices below sit just under and just
-over its lines (640 blocks at Ls = 12 and 16, 1300 at Ls = 8, 1500 for other Ls above
-10), with a ragged last block on each side, idle lanes (Ls = 5, 7, 10, 11, 12, 14, 18),
+over its lines for FP64 and FP32 hops (640 blocks at Ls = 12 and 16, 1300 at Ls = 8, 1200
+or 1500 above Ls = 10; test_gpu_hop_kernel.py has both kernels in every type), with a ragged last block on each side, idle lanes (Ls = 5, 7, 10, 11, 12, 14, 18),
 one and two matrix elements per thread (Ls = 16, 18), the largest Ls of the small kernel
 (22) and the first beyond it (23).  Bars as in the parity tests: FP64 1e-13, FP32 2e-6,
 FP16 4e-3, BF16 3e-2.
