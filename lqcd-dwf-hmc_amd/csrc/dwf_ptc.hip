@@ -838,6 +838,13 @@ static void ptc_layer_mfma_launch(float* out, const float* in, int cin, int cout
 #undef PTC_GO
 }
 
+// DWF_PTC_KERNEL: "valu" selects the VALU kernels everywhere, "valu-wgrad" only for the weight
+// gradients (the tests run them, and compare both gradients of the same layers)
+static bool ptc_valu(bool wgrad) {
+  const char* k = std::getenv("DWF_PTC_KERNEL");
+  return k && (std::strcmp(k, "valu") == 0 || (wgrad && std::strcmp(k, "valu-wgrad") == 0));
+}
+
 template <bool ADJ>
 static void ptc_layer_dispatch(float* out, const float* in, int cin, int cout, const unsigned* W,
                                int wcin, int wcout, const float* links, const int* nbr, int Vh,
@@ -845,11 +852,9 @@ static void ptc_layer_dispatch(float* out, const float* in, int cin, int cout, c
   // the matrix-core form (all output channels of 16 points per wave, an odd
   // count padded with a zero channel) wherever its 32-bit buffer offsets fit:
   // one channel's two parities, the links and the weights each below 2^31 bytes
-  // DWF_PTC_KERNEL=valu selects the VALU form everywhere (its tests use it)
   const size_t fsz = (size_t)Vh * 24 * Ls;
   const bool fits = 8 * fsz < (1ull << 31) && (size_t)2 * 8 * 18 * 4 * Vh < (1ull << 31);
-  const char* force = std::getenv("DWF_PTC_KERNEL");
-  if (fits && !(force && std::strcmp(force, "valu") == 0)) {
+  if (fits && !ptc_valu(false)) {
     switch ((cout + 1) / 2) {
 #define PTC_MFMA(n)                                                                          \
   case n:                                                                                    \
@@ -896,7 +901,7 @@ hipError_t launch_ptc_wgrad(double* G, double* partial, int maxblk, const float*
   // the other one's is that of cin cout (1290 and 181): they would be equal near 25 products
   // a tile group, and the line lies a little above.
   const int tb = ((cout + 1) / 2 + 3) / 4 * (((cin + 1) / 2 + 3) / 4);
-  if (Ls % 4 == 0 && cin * cout > 32 * tb) {
+  if (Ls % 4 == 0 && cin * cout > 32 * tb && !ptc_valu(true)) {
     // four 16-point groups a block until all maxblk blocks are there (with the 64 groups
     // that the other form takes, 8 -> 8 at 4^3 x 8, Ls = 8, had 44 blocks on 256 CUs)
     const int nblk = (int)std::max<size_t>(1, std::min<size_t>(maxblk, pts / 64));
