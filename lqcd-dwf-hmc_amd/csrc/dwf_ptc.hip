@@ -245,10 +245,12 @@ __device__ __forceinline__ void ptc_split_round(float x, float y, unsigned& hi, 
 // on an XCD then gather from two channels at a time, which its L2 holds between the nine
 // uses better than all of them.  The links of the wave's sites sit in LDS (they are read
 // once per pair), and so do the layer's weights where they fit (LW).  S16: Ls = 16, where
-// a tile is one site and the shifts in s are row shifts (DPP) of the split words.
+// a tile is one site and the shifts in s are row shifts (DPP) of the split words.  NB: the
+// channels of a pair that are loaded, 1 for cin = 1 (half the transports of the pair: 84 -> 76
+// us for the same network).
 constexpr int kPtcLinkDir = 20, kPtcLinkSite = 8 * kPtcLinkDir;   // floats in LDS
 __host__ __device__ constexpr int ptc_wave_sites(int Ls) { return 15 / Ls + 2; }
-template <bool ADJ, int NMT, bool LW, bool S16>
+template <bool ADJ, int NMT, bool LW, bool S16, int NB>
 __global__ void __launch_bounds__(256, NMT <= 2 ? 4 : NMT <= 5 ? 3 : 2)
 k_ptc_layer_mfma(float* __restrict__ out, const float* __restrict__ in, int cin, int cout,
                  const unsigned* __restrict__ W, int wcin, int wcout,
@@ -271,11 +273,6 @@ k_ptc_layer_mfma(float* __restrict__ out, const float* __restrict__ in, int cin,
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   float* su = reinterpret_cast<float*>(ptc_sw) + (size_t)wave * wsites * kPtcLinkSite;
   unsigned* sw = ptc_sw + (size_t)4 * wsites * kPtcLinkSite;
-  if (LW) {
-    for (int i = threadIdx.x; i < nwords / 4; i += 256)
-      reinterpret_cast<u32x4_t*>(sw)[i] = reinterpret_cast<const u32x4_t*>(W)[i];
-    __syncthreads();
-  }
   // the A row of this lane: channel 2 mt + am, spin row al, re (0) / im (1);
   // its weight word within the (q, b, mt) block
   const int am = n >> 3, al = (n >> 1) & 3, ro = n & 1;
@@ -286,21 +283,48 @@ k_ptc_layer_mfma(float* __restrict__ out, const float* __restrict__ in, int cin,
   const unsigned wlane =
       ADJ ? (unsigned)(am * 16 + g * 4 + al) : (unsigned)(am * wcin * 16 + al * 4 + g);
   // every XCD walks a contiguous range of sites: the neighbours of a tile share its L2
-  const int tile = xcd_block(blockIdx.x, gridDim.x) * 4 + wave;
-  if (tile >= 2 * tpp) return;
+  const int tile0 = xcd_block(blockIdx.x, gridDim.x) * 4 + wave;
+  const int tile = min(tile0, 2 * tpp - 1);
   const int p = tile / tpp;
   const int P0 = (tile - p * tpp) * 16, P = P0 + n;
   const bool valid = P < npts;
   const int Pc = valid ? P : npts - 1;
   const int site = Pc / Ls, s = Pc - (Pc / Ls) * Ls;
-  // links of sites site0 .. site0 + wsites - 1 (those below Vh), [site][dir][20]
-  const int site0 = P0 / Ls;
-  for (int i = lane; i < 144 * wsites; i += 64) {
-    const int r = i / wsites, j = i - r * wsites, d = r / 18;   // row = dir * 18 + e
-    const int x = site0 + j < Vh ? site0 + j : Vh - 1;
-    su[j * kPtcLinkSite + d * kPtcLinkDir + (r - 18 * d)] =
-        links[((size_t)p * 144 + r) * Vh + x];
+  // What every wave needs first, each in loads that are in flight together (one after the
+  // other they took most of a small lattice's time: 1 -> 3 -> 1 channels at 8^3 x 16, Ls = 12,
+  // 90 -> 84 us): the neighbours, the weights, the links of sites site0 .. site0 +
+  // wsites - 1 (those below Vh) as [site][dir][20].
+  int nb[8];
+#pragma unroll
+  for (int d = 0; d < 8; ++d) nb[d] = nbr[((size_t)p * 8 + d) * Vh + site];
+  if (LW) {
+    for (int i0 = threadIdx.x; i0 < nwords / 4; i0 += 4 * 256) {
+      u32x4_t v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        v[k] = reinterpret_cast<const u32x4_t*>(W)[min(i0 + 256 * k, nwords / 4 - 1)];
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        reinterpret_cast<u32x4_t*>(sw)[min(i0 + 256 * k, nwords / 4 - 1)] = v[k];
+    }
   }
+  const int site0 = P0 / Ls;
+  for (int i0 = lane; i0 < 144 * wsites; i0 += 5 * 64) {
+    float v[5];
+    int to[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      const int i = min(i0 + 64 * k, 144 * wsites - 1);
+      const int r = i / wsites, j = i - r * wsites, d = r / 18;   // row = dir * 18 + e
+      const int x = site0 + j < Vh ? site0 + j : Vh - 1;
+      v[k] = links[((size_t)p * 144 + r) * Vh + x];
+      to[k] = j * kPtcLinkSite + d * kPtcLinkDir + (r - 18 * d);
+    }
+#pragma unroll
+    for (int k = 0; k < 5; ++k) su[to[k]] = v[k];
+  }
+  if (LW) __syncthreads();
+  if (tile0 >= 2 * tpp) return;
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -311,8 +335,8 @@ k_ptc_layer_mfma(float* __restrict__ out, const float* __restrict__ in, int cin,
   off[0] = valid ? own : kOut;
 #pragma unroll
   for (int d = 0; d < 8; ++d) {
-    const int nb = nbr[((size_t)p * 8 + d) * Vh + site];
-    off[1 + d] = valid ? 4u * (unsigned)((1 - p) * fsz + ((size_t)nb * 24 + 6 * g) * Ls + s) : kOut;
+    off[1 + d] = 4u * (unsigned)((1 - p) * fsz + ((size_t)nb[d] * 24 + 6 * g) * Ls + s);
+    if (!valid) off[1 + d] = kOut;
   }
   off[9] = valid && s + 1 < Ls ? own + 4u : kOut;
   off[10] = valid && s > 0 ? own - 4u : kOut;
@@ -328,11 +352,11 @@ k_ptc_layer_mfma(float* __restrict__ out, const float* __restrict__ in, int cin,
     const __amdgpu_buffer_rsrc_t r0 = ptc_rsrc(in + (size_t)b * 2 * fsz, 8u * (unsigned)fsz);
     const __amdgpu_buffer_rsrc_t r1 =
         ptc_rsrc(in + (size_t)(two ? b + 1 : b) * 2 * fsz, two ? 8u * (unsigned)fsz : 0u);
-    auto load = [&](int q, float (&w)[2][6]) {
+    auto load = [&](int q, float (&w)[NB][6]) {
 #pragma unroll
-      for (int k = 0; k < 6; ++k) w[0][k] = ptc_ld(r0, off[q], (unsigned)k * lsb);
+      for (int j = 0; j < NB; ++j)
 #pragma unroll
-      for (int k = 0; k < 6; ++k) w[1][k] = ptc_ld(r1, off[q], (unsigned)k * lsb);
+        for (int k = 0; k < 6; ++k) w[j][k] = ptc_ld(j ? r1 : r0, off[q], (unsigned)k * lsb);
     };
     // element (al, beta = g) of the applied spin matrix of channel a = 2 mt + am:
     // forward W[qw][a][b], adjoint (W[qw][b][a])^+, as the coefficients of (re, im);
@@ -343,6 +367,10 @@ k_ptc_layer_mfma(float* __restrict__ out, const float* __restrict__ in, int cin,
       for (int mt = 0; mt < NMT; ++mt)
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
+          if (j >= NB) {
+            A[mt][j] = 0u;
+            continue;
+          }
           const unsigned wblk = ADJ ? (unsigned)(((qw * wcout + b + j) * wcin + 2 * mt) * 16)
                                     : (unsigned)(((qw * wcout + 2 * mt) * wcin + b + j) * 16);
           const bool on = (j == 0 || two) && 2 * mt + am < cout;
@@ -374,23 +402,23 @@ k_ptc_layer_mfma(float* __restrict__ out, const float* __restrict__ in, int cin,
       B[2][j] = hi;
     };
     // paths without a link
-    auto plain = [&](int q, const float (&w)[2][6]) {
+    auto plain = [&](int q, const float (&w)[NB][6]) {
       ptc_w2_t A[NMT];
       weights(q, A);
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
-        ptc_w2_t B[3];
+        ptc_w2_t B[3] = {};
 #pragma unroll
-        for (int j = 0; j < 2; ++j) split(w[j][2 * c], w[j][2 * c + 1], B, j);
+        for (int j = 0; j < NB; ++j) split(w[j][2 * c], w[j][2 * c + 1], B, j);
         products(A, B, c);
         if constexpr (S16) {   // s + 1 and s - 1: the neighbouring lanes, 0 beyond the walls
-          ptc_w2_t U[3], D[3], Au[NMT], Ad[NMT];
+          ptc_w2_t U[3] = {}, D[3] = {}, Au[NMT], Ad[NMT];
           weights(9, Au);
           weights(10, Ad);
 #pragma unroll
           for (int part = 0; part < 3; ++part)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
+            for (int j = 0; j < NB; ++j) {
               U[part][j] = __builtin_amdgcn_update_dpp(0, (int)B[part][j], 0x101, 0xf, 0xf, true);
               D[part][j] = __builtin_amdgcn_update_dpp(0, (int)B[part][j], 0x111, 0xf, 0xf, true);
             }
@@ -401,7 +429,7 @@ k_ptc_layer_mfma(float* __restrict__ out, const float* __restrict__ in, int cin,
     };
     // a hop: colour by colour the transported component of spin g at this point, both
     // channels, split, then its products
-    auto hop = [&](int q, const float (&w)[2][6]) {
+    auto hop = [&](int q, const float (&w)[NB][6]) {
       ptc_w2_t A[NMT];
       weights(q, A);
       float u[18];
@@ -409,9 +437,9 @@ k_ptc_layer_mfma(float* __restrict__ out, const float* __restrict__ in, int cin,
       for (int e = 0; e < 18; ++e) u[e] = ul[(q - 1) * kPtcLinkDir + e];
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
-        ptc_w2_t B[3];
+        ptc_w2_t B[3] = {};
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < NB; ++j) {
           float re = 0.f, im = 0.f;
 #pragma unroll
           for (int cb = 0; cb < 3; ++cb)
@@ -422,7 +450,7 @@ k_ptc_layer_mfma(float* __restrict__ out, const float* __restrict__ in, int cin,
         products(A, B, c);
       }
     };
-    float wa[2][6], wb[2][6];
+    float wa[NB][6], wb[NB][6];
     load(0, wa);
     if constexpr (S16) {
       load(1, wb); plain(0, wa);
@@ -835,13 +863,16 @@ static void ptc_layer_mfma_launch(float* out, const float* in, int cin, int cout
   const size_t lbytes = (size_t)4 * ptc_wave_sites(Ls) * kPtcLinkSite * sizeof(float);
   const dim3 grid((unsigned)((tiles + 3) / 4)), block(256);
   const bool lw = lbytes + wbytes <= 64 * 1024 && reinterpret_cast<uintptr_t>(W) % 16 == 0;
-#define PTC_GO(L, S)                                                                          \
-  hipLaunchKernelGGL((k_ptc_layer_mfma<ADJ, NMT, L, S>), grid, block, lbytes + (L ? wbytes : 0), \
-                     st, out, in, cin, cout, W, wcin, wcout, links, nbr, Vh, Ls)
-  if (lw && Ls == 16) PTC_GO(true, true);
-  else if (lw) PTC_GO(true, false);
-  else if (Ls == 16) PTC_GO(false, true);
-  else PTC_GO(false, false);
+#define PTC_GO(L, S, NB)                                                                      \
+  hipLaunchKernelGGL((k_ptc_layer_mfma<ADJ, NMT, L, S, NB>), grid, block,                     \
+                     lbytes + (L ? wbytes : 0), st, out, in, cin, cout, W, wcin, wcout, links, nbr, \
+                     Vh, Ls)
+  if (lw && cin == 1 && Ls == 16) PTC_GO(true, true, 1);
+  else if (lw && cin == 1) PTC_GO(true, false, 1);
+  else if (lw && Ls == 16) PTC_GO(true, true, 2);
+  else if (lw) PTC_GO(true, false, 2);
+  else if (Ls == 16) PTC_GO(false, true, 2);
+  else PTC_GO(false, false, 2);
 #undef PTC_GO
 }
 
