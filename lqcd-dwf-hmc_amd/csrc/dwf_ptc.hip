@@ -28,6 +28,7 @@
 namespace dwf {
 
 constexpr int kPtcPaths = 11;
+constexpr int kPtcLinkDir = 20, kPtcLinkSite = 8 * kPtcLinkDir;   // links of a site in LDS, floats
 
 // (re, im) += (ar + i ai)(br + i bi), two fused multiply-adds per part
 __device__ __forceinline__ void cmac(float& re, float& im, float ar, float ai, float br,
@@ -169,10 +170,22 @@ __device__ __forceinline__ float ptc_ld(__amdgpu_buffer_rsrc_t r, unsigned voff,
 typedef unsigned ptc_w2_t __attribute__((ext_vector_type(2)));
 typedef short ptc_s4_t __attribute__((ext_vector_type(4)));
 
-// t = hi + mid + lo exactly, each part with at most 8 significant bits, i.e. a
-// bfloat16 (the first sixteen bits of its float): truncate, subtract, truncate.  The
-// parts of (re, im) are returned as one word each, re low; the subtraction takes its
-// part from the word (v_dot2_f32_bf16 with (-1, 0) and (0, -1), exact here).
+// The splits below are exact where every part is a bfloat16, denormals (multiples of 2^-133)
+// included: for finite numbers from about 2^-109 up.  Smaller ones lose their last bits, and
+// an infinity leaves inf - inf (with rounded parts a number beyond the largest bfloat16, too).
+// So a tile whose sums hold a NaN, or in a lane nothing but numbers so small that they can
+// stem from such transports, is formed again in FP32; what is lost in the others is below
+// 2^-133 beside sums of at least 2^-88.
+constexpr float kPtcTiny = 0x1p-88f;
+__device__ __forceinline__ float ptc_absmax(float m, float x, float y) {   // NaN stays
+  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, fabsf(x)), fabsf(y));
+}
+__device__ __forceinline__ bool ptc_in_range(float m) { return m == 0.f || m >= kPtcTiny; }
+
+// t = hi + mid + lo, each part with at most 8 significant bits, i.e. a bfloat16 (the first
+// sixteen bits of its float): truncate, subtract, truncate.  The parts of (re, im) are
+// returned as one word each, re low; the subtraction takes its part from the word
+// (v_dot2_f32_bf16 with (-1, 0) and (0, -1), exact here).
 __device__ __forceinline__ void ptc_split(float re, float im, unsigned& hi, unsigned& mid,
                                           unsigned& lo) {
   typedef __bf16 b2_t __attribute__((ext_vector_type(2)));
@@ -194,8 +207,7 @@ __device__ __forceinline__ void ptc_split(float re, float im, unsigned& hi, unsi
 }
 
 // The same split with rounded parts (their signs are then as good as random, so that a
-// dropped product of parts leaves no bias); a float within half a bfloat16 step of the
-// largest becomes infinite.
+// dropped product of parts leaves no bias).
 __device__ __forceinline__ void ptc_split_round(float x, float y, unsigned& hi, unsigned& mid,
                                                 unsigned& lo) {
   typedef __bf16 b2_t __attribute__((ext_vector_type(2)));
@@ -213,6 +225,98 @@ __device__ __forceinline__ void ptc_split_round(float x, float y, unsigned& hi, 
   hi = __builtin_bit_cast(unsigned, h);
   mid = __builtin_bit_cast(unsigned, m);
   lo = __builtin_bit_cast(unsigned, l);
+}
+
+// a tile's sums to the output: register r of lane (n, g) is row 4 g + r = channel
+// 2 mt + (g >> 1), spin 2 (g & 1) + (r >> 1), re / im r & 1, of point n
+template <int NMT>
+__device__ __forceinline__ void ptc_tile_store(float* out, const flt4_t (&acc)[NMT][3], int cout,
+                                               size_t fsz, int p, int site, int s, int g, int Ls) {
+#pragma unroll
+  for (int mt = 0; mt < NMT; ++mt) {
+    if (2 * mt + (g >> 1) >= cout) continue;
+    float* o = out + (size_t)(2 * mt + (g >> 1)) * 2 * fsz + (size_t)p * fsz +
+               (size_t)site * 24 * Ls + s;
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int alo = 2 * (g & 1) + (r >> 1);
+        o[(size_t)((r & 1) + 2 * (c + 3 * alo)) * Ls] = acc[mt][c][r];
+      }
+  }
+}
+
+// One tile of k_ptc_layer_mfma again on the FP32 matrix cores, for transports outside the range
+// of the split: D(16x16) += A(16x4) B(4x16), K the 4 spins, t_re and t_im in turn.  A function
+// of its own: inlined, its registers cost the layers where it never runs (8.9 ms an application
+// at 16^3 x 32, Ls = 16, against 8.65; 8.55 without the check).
+template <bool ADJ, int NMT>
+__device__ __attribute__((noinline)) void ptc_tile_f32(
+    float* out, const float* in, int cin, int cout, const unsigned* W, int wcin, int wcout,
+    const float* su, const int* nbr, int Vh, int Ls, int tile) {
+  constexpr unsigned kOut = 0x80000000u;
+  const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+  const int am = n >> 3, al = (n >> 1) & 3, ro = n & 1;   // as in k_ptc_layer_mfma
+  const size_t fsz = (size_t)Vh * 24 * Ls;
+  const int npts = Vh * Ls, tpp = (npts + 15) / 16, p = tile / tpp;
+  const int P0 = (tile - p * tpp) * 16;
+  const bool valid = P0 + n < npts;
+  const int P = valid ? P0 + n : npts - 1, site = P / Ls, s = P - site * Ls;
+  const float* ul = su + (site - P0 / Ls) * kPtcLinkSite;
+  const __amdgpu_buffer_rsrc_t rw = ptc_rsrc(W, 4u * (unsigned)(kPtcPaths * wcin * wcout * 16));
+  flt4_t acc[NMT][3];
+#pragma unroll
+  for (int mt = 0; mt < NMT; ++mt)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) acc[mt][c] = flt4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int q = 0; q < kPtcPaths; ++q) {
+    const int qw = ADJ ? ptc_rev(q) : q;
+    const bool hop = q >= 1 && q <= 8;
+    const int ss = s + (q == 9) - (q == 10);
+    const int x = hop ? nbr[((size_t)p * 8 + q - 1) * Vh + site] : site;
+    const unsigned off =
+        valid && ss >= 0 && ss < Ls
+            ? 4u * (unsigned)((hop ? 1 - p : p) * fsz + ((size_t)x * 24 + 6 * g) * Ls + ss)
+            : kOut;
+#pragma unroll 1
+    for (int b = 0; b < cin; ++b) {
+      const __amdgpu_buffer_rsrc_t r = ptc_rsrc(in + (size_t)b * 2 * fsz, 8u * (unsigned)fsz);
+      float w[6], t[6];
+#pragma unroll
+      for (int k = 0; k < 6; ++k) w[k] = t[k] = ptc_ld(r, off, 4u * (unsigned)(k * Ls));
+      if (hop) {
+        const float* u = ul + (q - 1) * kPtcLinkDir;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          float re = 0.f, im = 0.f;
+#pragma unroll
+          for (int cb = 0; cb < 3; ++cb)
+            cmac(re, im, u[2 * (cb + 3 * c)], u[2 * (cb + 3 * c) + 1], w[2 * cb], w[2 * cb + 1]);
+          t[2 * c] = re;
+          t[2 * c + 1] = im;
+        }
+      }
+#pragma unroll
+      for (int mt = 0; mt < NMT; ++mt) {
+        const unsigned wblk = ADJ ? (unsigned)(((qw * wcout + b) * wcin + 2 * mt) * 16)
+                                  : (unsigned)(((qw * wcout + 2 * mt) * wcin + b) * 16);
+        const unsigned wl = ADJ ? (unsigned)(am * 16 + g * 4 + al)
+                                : (unsigned)(am * wcin * 16 + al * 4 + g);
+        const unsigned e = ptc_ldu(rw, 2 * mt + am < cout ? 4u * wl : kOut, 4u * wblk);
+        const float wr = __uint_as_float(e << 16);
+        const float wi = ADJ ? -__uint_as_float(e & 0xffff0000u) : __uint_as_float(e & 0xffff0000u);
+        const float ar = ro ? wi : wr, ai = ro ? wr : -wi;   // multiply t_re, t_im
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          acc[mt][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(ar, t[2 * c], acc[mt][c], 0, 0, 0);
+          acc[mt][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(ai, t[2 * c + 1], acc[mt][c], 0, 0, 0);
+        }
+      }
+    }
+  }
+  if (valid) ptc_tile_store<NMT>(out, acc, cout, fsz, p, site, s, g, Ls);
 }
 
 // Matrix-core form of the same layer (any number of output channels up to 16;
@@ -248,7 +352,6 @@ __device__ __forceinline__ void ptc_split_round(float x, float y, unsigned& hi, 
 // a tile is one site and the shifts in s are row shifts (DPP) of the split words.  NB: the
 // channels of a pair that are loaded, 1 for cin = 1 (half the transports of the pair: 84 -> 76
 // us for the same network).
-constexpr int kPtcLinkDir = 20, kPtcLinkSite = 8 * kPtcLinkDir;   // floats in LDS
 __host__ __device__ constexpr int ptc_wave_sites(int Ls) { return 15 / Ls + 2; }
 template <bool ADJ, int NMT, bool LW, bool S16, int NB>
 __global__ void __launch_bounds__(256, NMT <= 2 ? 4 : NMT <= 5 ? 3 : 2)
@@ -470,23 +573,19 @@ k_ptc_layer_mfma(float* __restrict__ out, const float* __restrict__ in, int cin,
     hop(7, wb);
     hop(8, wa);
   }
-  if (valid) {
-    // register r: row 4 g + r = channel 2 mt + (g >> 1), spin 2 (g & 1) + (r >> 1),
-    // re / im r & 1
+  float m = 0.f;
 #pragma unroll
-    for (int mt = 0; mt < NMT; ++mt) {
-      if (2 * mt + (g >> 1) >= cout) continue;
-      float* o = out + (size_t)(2 * mt + (g >> 1)) * 2 * fsz + (size_t)p * fsz +
-                 (size_t)site * 24 * Ls + s;
+  for (int mt = 0; mt < NMT; ++mt)
 #pragma unroll
-      for (int c = 0; c < 3; ++c)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int alo = 2 * (g & 1) + (r >> 1);
-          o[(size_t)((r & 1) + 2 * (c + 3 * alo)) * Ls] = acc[mt][c][r];
-        }
+    for (int c = 0; c < 3; ++c) {
+      m = ptc_absmax(m, acc[mt][c][0], acc[mt][c][1]);
+      m = ptc_absmax(m, acc[mt][c][2], acc[mt][c][3]);
     }
+  if (__builtin_expect(__ballot(!ptc_in_range(m)) != 0, 0)) {
+    ptc_tile_f32<ADJ, NMT>(out, in, cin, cout, W, wcin, wcout, su, nbr, Vh, Ls, tile);
+    return;
   }
+  if (valid) ptc_tile_store<NMT>(out, acc, cout, fsz, p, site, s, g, Ls);
 }
 
 // Weight gradient of one layer: block (x, y = q * cin + b, z) adds, over its
@@ -552,6 +651,49 @@ k_ptc_wgrad(double* __restrict__ partial, const float* __restrict__ g,
                      sh[3][threadIdx.x];
     partial[(((size_t)blockIdx.y * cout + a0 + j) * gridDim.x + blockIdx.x) * 32 + k] = v;
   }
+}
+
+// One block's part of the weight gradient of output channel a and input channel b again, in
+// FP32, for k_ptc_wgrad_mfma: the points of its groups first .. last - 1; sh 128 doubles.
+__device__ __forceinline__ void ptc_wgrad_f32(double* dst, const float* __restrict__ g,
+                              const float* __restrict__ in, int a, int b,
+                              const float* __restrict__ links, const int* __restrict__ nbr, int q,
+                              int first, int last, int Vh, int Ls, double* sh) {
+  const size_t fsz = (size_t)Vh * 24 * Ls;
+  const int npts = Vh * Ls, gpp = (npts + 15) / 16;
+  float acc[32];
+#pragma unroll
+  for (int k = 0; k < 32; ++k) acc[k] = 0;
+  for (int i = 16 * first + (int)threadIdx.x; i < 16 * last; i += 256) {
+    const int p = i >= 16 * gpp ? 1 : 0, P = i - p * 16 * gpp;
+    if (P >= npts) continue;
+    const int site = P / Ls, s = P - site * Ls;
+    float t[24];
+    if (!ptc_transport(t, in + (size_t)b * 2 * fsz, links, nbr, q, p, site, s, Vh, Ls)) continue;
+    const float* gp = g + ((size_t)a * 2 + p) * fsz + (size_t)site * 24 * Ls + s;
+#pragma unroll
+    for (int al = 0; al < 4; ++al)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const float gr = gp[(6 * al + 2 * c) * Ls], gi = gp[(6 * al + 2 * c + 1) * Ls];
+#pragma unroll
+        for (int be = 0; be < 4; ++be)   // g conj(t)
+          cmac(acc[2 * (al * 4 + be)], acc[2 * (al * 4 + be) + 1], gr, gi, t[2 * (c + 3 * be)],
+               -t[2 * (c + 3 * be) + 1]);
+      }
+  }
+#pragma unroll
+  for (int k = 0; k < 32; ++k) {
+    double v = acc[k];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+    if ((threadIdx.x & 63) == 0) sh[(threadIdx.x >> 6) * 32 + k] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x < 32)
+    dst[threadIdx.x] = sh[threadIdx.x] + sh[32 + threadIdx.x] + sh[64 + threadIdx.x] +
+                       sh[96 + threadIdx.x];
+  __syncthreads();
 }
 
 // The same for Ls a multiple of 4 on the matrix cores: per path one real product
@@ -654,6 +796,8 @@ k_ptc_wgrad_mfma(double* __restrict__ partial, const float* __restrict__ gr,
       for (int c = 0; c < 3; ++c) edge[c] = s > 0 ? (x + c * step)[-1] : 0.f;
     }
   };
+  // largest operands of this lane, one colour's for all (every sum runs over the colours)
+  float max_a = 0.f, max_b = 0.f;
   auto parts = [&](flt4_t v, unsigned (&hi)[2], unsigned (&mid)[2], unsigned (&lo)[2]) {
     ptc_split_round(v[0], v[1], hi[0], mid[0], lo[0]);
     ptc_split_round(v[2], v[3], hi[1], mid[1], lo[1]);
@@ -675,6 +819,7 @@ k_ptc_wgrad_mfma(double* __restrict__ partial, const float* __restrict__ gr,
         parts(va[c], hi, mid, lo);
         put(shA + (wave * 3 + c) * 192 + lane, hi, mid, lo);
       }
+      max_a = ptc_absmax(ptc_absmax(max_a, va[0][0], va[0][1]), va[0][2], va[0][3]);
     }
     if (colt) {
       flt4_t x[3];
@@ -712,6 +857,7 @@ k_ptc_wgrad_mfma(double* __restrict__ partial, const float* __restrict__ gr,
         parts(x[c], hi, mid, lo);
         put(shB + (wave * 3 + c) * 192 + lane, hi, mid, lo);
       }
+      max_b = ptc_absmax(ptc_absmax(max_b, x[0][0], x[0][1]), x[0][2], x[0][3]);
     }
   };
   const int tr = 2 * (wave >> 1), tc = 2 * (wave & 1);   // this wave's quadrant
@@ -774,6 +920,18 @@ k_ptc_wgrad_mfma(double* __restrict__ partial, const float* __restrict__ gr,
           for (int r = 0; r < 4; ++r) acc[i][j][r] = fma(sign, (double)d[i][j][r], acc[i][j][r]);
     }
     __syncthreads();
+  }
+  if (__syncthreads_or(!ptc_in_range(max_a) || !ptc_in_range(max_b))) {
+    // outside the range of the split: this block's points in FP32, pair by pair
+    double* sh = reinterpret_cast<double*>(shA);
+    const int a1 = min(2 * rt0 + 8, cout), b1 = min(2 * ct0 + 8, cin);
+#pragma unroll 1
+    for (int gb = 2 * ct0; gb < b1; ++gb)
+#pragma unroll 1
+      for (int ga = 2 * rt0; ga < a1; ++ga)
+        ptc_wgrad_f32(partial + (((size_t)(q * cin + gb) * cout + ga) * gridDim.x + blockIdx.x) * 32,
+                      gr, in, ga, gb, links, nbr, q, first, last, Vh, Ls, sh);
+    return;
   }
   // P -> g conj(t): the lane of t_re holds (g_re, g_im) t_re in registers 2 k, 2 k + 1, its
   // neighbour those of t_im;  re = g_re t_re + g_im t_im,  im = g_im t_re - g_re t_im
