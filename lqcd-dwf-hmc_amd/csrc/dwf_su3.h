@@ -209,6 +209,10 @@ template <> struct M3Pipe<true> {
   // the first two matrices
   __device__ __forceinline__ void start(const double* b0, int s0, const double* b1, int s1) {
     issue<0>(b0, s0);
+    // take() counts loads: slot 0's must be the older ones, and to the compiler the two
+    // slots are unrelated memory
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
     issue<1>(b1, s1);
   }
   // this lane's row of a slot once at most YOUNGER loads are outstanding.  One
