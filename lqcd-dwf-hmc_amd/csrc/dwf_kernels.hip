@@ -1226,7 +1226,11 @@ static hipError_t launch_combo(int op, bool mat, bool addx, bool out2, dim3 g, d
     } else {
       LK(K_SITE, true, false, false);
     }
-  } else if (op == K_HOP) {
+    return hipGetLastError();
+  }
+  // Ls = 4: site launches only (dwf_shape_t)
+  if constexpr (LSC == 4) return hipErrorInvalidValue;
+  else if (op == K_HOP) {
     if (!mat) {
       if (addx || out2) return hipErrorInvalidValue;
       LK(K_HOP, false, false, false);
@@ -1273,7 +1277,10 @@ static hipError_t dwf_shape_t(int op, const void* out, int Ls, const Epi& e, Dwf
   if (op == K_HOPDAG && out2 && !addx) return hipErrorInvalidValue;
   if ((e.G && !addx) || (e.X2 && !out2)) return hipErrorInvalidValue;
   const int vec = KCfg<T>::VEC;
-  shape->lsc = (Ls == 4 || Ls == 8 || Ls == 12 || Ls == 16) && Ls % vec == 0;
+  // compiled Ls; at Ls = 4 the FP64 and FP32 site launches alone, the rest goes to k_dwf_small
+  // at every volume (and a block of hops would not fit in LDS)
+  shape->lsc = (Ls == 8 || Ls == 12 || Ls == 16 || (Ls == 4 && op == K_SITE && sizeof(T) > 2)) &&
+               Ls % vec == 0;
   int spb = shape->lsc ? spb_of<T>(Ls, vec) : KCfg<T>::THREADS / Ls;
   if (spb < 1) return hipErrorInvalidValue;
   const size_t cs = sizeof(C);
@@ -1287,9 +1294,8 @@ static hipError_t dwf_shape_t(int op, const void* out, int Ls, const Epi& e, Dwf
     const size_t epi = mat ? (size_t)sp * (mfma_ls(Ls) && shape->lsc ? 12 * 17 : 2 * (12 * Ls + 1)) * cs : 0;
     return (stage > epi ? stage : epi) + matb;
   };
-  // The compiled-Ls kernels fix their block at THREADS / (Ls / VEC) sites; when
-  // that block's link staging exceeds the LDS cap (FP64 and FP32 at Ls = 4) the
-  // runtime-Ls kernel runs instead, with fewer sites per block.
+  // The compiled-Ls kernels fix their block at THREADS / (Ls / VEC) sites; the runtime-Ls
+  // kernel takes as many as fit.
   // the fused CG updates, and an output that is not stored, exist in the
   // matrix-core epilogue only
   const bool mfma_path = mat && mfma_ls(Ls) && shape->lsc && lds_for(spb) <= lds_cap;
@@ -1322,12 +1328,11 @@ static hipError_t launch_dwf_t(const DwfShape& sh, int op, void* out, const void
   return launch_combo<T, L>(op, mat, addx, out2, grid, block, sh.lds, st, out, in, links, nbr,  \
                             parity, Vh, Ls, sh.spb, e)
   if (!sh.lsc) LC(0);
-  switch (Ls) {
-    case 4: LC(4);
-    case 8: LC(8);
-    case 12: LC(12);
-    default: LC(16);
-  }
+  if (Ls == 8) LC(8);
+  if (Ls == 12) LC(12);
+  if (Ls == 16) LC(16);
+  if constexpr (sizeof(T) > 2) LC(4);
+  return hipErrorInvalidValue;
 #undef LC
 }
 

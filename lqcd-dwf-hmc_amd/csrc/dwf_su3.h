@@ -138,16 +138,6 @@ __device__ __forceinline__ M3 m3_zero() {
   return r;
 }
 
-__device__ __forceinline__ M3 dag3(const M3& x) {
-  M3 r;
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) r.a[i][j] = {x.a[j][i].r, -x.a[j][i].i};
-  return r;
-}
-
-// anti-hermitian traceless part: at(m) = (m - m^+)/2 - tr(m - m^+)/6
 __device__ __forceinline__ M3 at3(const M3& m) {
   M3 r;
 #pragma unroll
