@@ -325,7 +325,7 @@ __device__ __attribute__((noinline)) void ptc_tile_f32(
 // real product
 //   [out_re; out_im](a, alpha) += [Wr -Wi; Wi Wr](a, alpha; beta) [t_re; t_im](beta)
 // for every colour.  The weights are bfloat16, and the FP32 transports are the exact sum
-// of three bfloat16 parts, so the products run on the BF16 matrix cores without loss
+// of three bfloat16 parts (ptc_split), so the products run on the BF16 matrix cores without loss
 // (v_mfma_f32_16x16x16_bf16, FP32 accumulation): 3 x 16 cycles per tile, colour and two
 // input channels where the FP32 cores take 4 x 32.  Tiles D(16x16) += A(16x16) B(16x16) with
 //   D rows  m = 8 a' + 2 alpha + re/im  (NMT tiles of two output channels),
@@ -338,9 +338,9 @@ __device__ __attribute__((noinline)) void ptc_tile_f32(
 // row; register r of its result holds D[4 (l / 16) + r][l % 16].  One wave
 // per 16 points, all output channels; each output element is a sum over
 // (q, b pairs, parts) of 8-term matrix-core products in FP32.
-// 1 -> 8 -> 8 -> 8 -> 1 channels at 16^3 x 32, Ls = 16: 13.5 -> 8.8 ms (error against
+// 1 -> 8 -> 8 -> 8 -> 1 channels at 16^3 x 32, Ls = 16: 13.5 -> 8.7 ms (error against
 // 64 bits 9.5e-7 -> 6e-7).  Bound by the gathers: every channel is read nine times through
-// L1 (14.5 GB per 8 -> 8 layer, 12.6 GB of it past the L2s); the vector unit has 1.4 ms
+// L1 (14.5 GB per 8 -> 8 layer, 9.9 GB of it past the L2s); the vector unit has 1.4 ms
 // of work per such layer (36 operations of transport and 21 of splitting per hop path
 // and channel), the matrix cores 1.35 ms.  Two s per lane with eight-byte loads (9.9 ms),
 // all channels per path (9.9) and no per-XCD order (9.6, before the shifts by lane, against

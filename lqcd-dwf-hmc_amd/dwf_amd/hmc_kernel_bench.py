@@ -2,10 +2,11 @@
 kernel traces and hardware counters, and prints the algorithmic bytes of one
 launch of each (what the kernel must read and write once):
 
-* k_stout               one stout level: read U, write U' (gauge field = 4 V 18 doubles)
+* k_gauge_chunk         the thin links copied to the chunked form (gauge field = 4 V 18 doubles)
+* k_stout               one stout level: read U, write U' and, but for the last, its chunked copy
 * k_stout_force_link    per level: read U, Sigma'; write Sigma, iTheta
 * k_stout_force_staple  per level: read U, iTheta, Sigma; write Sigma
-* k_force_tensor        two 5D half spinors, read and write the force rows of one parity
+* k_force_tensor        one term (force_udiv1): four 5D half spinors read, the force written
 * k_shift_update_all    16 shifts: shifts 1..15 (x_j, p_j read and written, r read once;
                         shift 0 is the unshifted CG's own x, p)
 * k_rect_force          read U, write F
@@ -49,7 +50,8 @@ def main():
     for _ in range(reps):
         sm.set_config(U0)
     dwf_amd.synchronize()
-    print(f"k_stout: {2 * G} B per launch (3 per set_config)", flush=True)
+    print(f"k_gauge_chunk: {2 * G} B per launch, k_stout: {3 * G} B (2 of 3 per set_config), "
+          f"{2 * G} B (the last)", flush=True)
 
     op = dwf_amd.AFopr_Domainwall_5din_eo(dims, Ls, 0.01, 1.0, 1.5, 0.5, (1, 1, 1, -1), "double")
     op.set_config_smeared(sm, None)
@@ -62,7 +64,7 @@ def main():
     for _ in range(reps):
         force.force_udiv1(F, zeta, eta)
     dwf_amd.synchronize()
-    print(f"k_force_tensor: {2 * half + G} B per launch (2 per force_udiv1)", flush=True)
+    print(f"k_force_tensor: {4 * half + G} B per launch (1 per force_udiv1)", flush=True)
     for _ in range(reps):
         for level in (2, 1, 0):
             sm.force_udiv(F, F, level)
