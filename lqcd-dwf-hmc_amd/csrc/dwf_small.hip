@@ -291,6 +291,10 @@ static size_t small_lds(int prec, int op, int Ls, const Epi& e) {
 //   (5462 14.2 / 21.1).
 // * larger Ls: the transposed matrices take LDS, and from Ls = 17 on lanes idle: FP16 site
 //   Ls = 14 1024 7.3 / 6.5, 3456 10.9 / 16.1; hop FP16 Ls = 22 2048 28 / 20, 6912 47 / 58.
+// 16-bit storage at Ls = 12 and 16 keeps the hops' line for its sites, too: k_dwf rounds the
+// operands of its matrix-core epilogue to the storage type, this kernel does not (FP16 D_ee^-1
+// errors 4.0e-4 and 2.9e-4), and that is worth more than the microsecond or two it takes longer
+// between (site BF16 Ls = 16 1024 5.0 / 6.7).
 // A hop without E lacks the epilogue that this kernel spreads over its waves, and a site
 // launch the gathers: both leave it earlier than a hop does.
 static long small_max_blocks(int prec, int op, bool mat, int Ls) {
@@ -300,7 +304,8 @@ static long small_max_blocks(int prec, int op, bool mat, int Ls) {
     if (Ls == 4) return f64 ? 600 : f32 ? 1000 : all;
     if (Ls == 8) return f64 ? 600 : f32 ? 900 : 1200;
     if (Ls == 10) return b16 ? 2000 : all;
-    if (Ls == 12) return b16 ? 1000 : 400;
+    if ((Ls == 12 || Ls == 16) && b16) return prec == PBF16 ? 1500 : 640;
+    if (Ls == 12) return 400;
     if (Ls == 16) return f64 ? 250 : 400;
     return Ls <= 11 ? all : f64 ? 1500 : 1100;
   }

@@ -3,7 +3,8 @@ are never read).
 
 What it accepts does not depend on the volume: the forms that k_dwf refuses are refused on a
 small lattice too, where k_dwf_small would run.  And which of the two kernels a launch takes
-follows what either one was measured to take."""
+follows what either one was measured to take (but for 16-bit sites at Ls = 12 and 16, where
+k_dwf rounds more)."""
 import os
 import shutil
 import subprocess
@@ -61,7 +62,7 @@ P32 10 36864 hop 355.6 331.9  P16 6 33178 site 179.9 105.2  P64 6 9831 hop 155.1
 P16 10 5462 site 14.2 21.1    P16 14 1024 site 7.3 6.5      P16 14 3456 site 10.9 16.1
 P16 22 2048 hop 28.1 20.4     P16 22 6912 hop 47.1 58.4     P16 20 6912 scalar 29.3 35.3
 P64 9 2963 scalar 36.8 47.0   P32 4 4096 site 11.9 15.9     P64 4 2560 site 11.0 13.4
-PBF16 16 1024 site 5.0 6.7    P16 22 3600 scalar 19.5 22.5  P16 4 4096 site 15.9 14.7
+P16 22 3600 scalar 19.5 22.5  P16 4 4096 site 15.9 14.7
 """
 
 RULE = r"""
